@@ -233,7 +233,8 @@ int uc_kivi_attn_decode(const uc_kivi_item *item_host, int bits, int group_size,
  * GPU's scratch: calls that overlap on one GPU (different streams or host
  * threads without ordering) race and give wrong results.  The device current
  * on the calling thread must be the one that owns the item's tensors and
- * `stream`.  Results equal uc_kivi_attn_decode's bit for bit.
+ * `stream`.  Results equal bit for bit those of uc_kivi_attn_decode with a
+ * workspace of uc_kivi_decode_workspace_bytes(1, ...) bytes.
  */
 int uc_kivi_attn_decode_static(const uc_kivi_item *item_host, int bits, int group_size,
                                int64_t heads_q, int64_t heads_kv, int64_t head_dim, int64_t query_len,
@@ -663,6 +664,17 @@ int64_t uc_workspace_bytes(int op, int64_t n_items, int64_t heads_q, int64_t que
 int64_t uc_kivi_decode_workspace_bytes(int64_t n_items, int bits, int group_size, int64_t heads_q,
                                        int64_t heads_kv, int64_t head_dim, int64_t query_len,
                                        int64_t max_quantized_tokens, int64_t max_residual_tokens);
+
+/*
+ * Bytes of workspace with which the same calls are fastest: launches too small
+ * to fill the GPU then split their segments finer, into more partials.  At
+ * least uc_kivi_decode_workspace_bytes and at most about 3.3 MB more.  A call
+ * with less workspace than this is valid and splits coarser; its results
+ * differ in the rounding of the partials only.
+ */
+int64_t uc_kivi_decode_preferred_workspace_bytes(int64_t n_items, int bits, int group_size, int64_t heads_q,
+                                                 int64_t heads_kv, int64_t head_dim, int64_t query_len,
+                                                 int64_t max_quantized_tokens, int64_t max_residual_tokens);
 
 #ifdef __cplusplus
 }

@@ -90,6 +90,17 @@ def test_workspace_bytes():
         nat.workspace_bytes(99, 1, 1, 1, 1, 1)
 
 
+def test_preferred_decode_workspace():
+    # room for splits of one super-tile, up to one round of 768 workgroups; never less than the call needs
+    slot = 16 * 128 * 2 + 16 * 2 * 4
+    assert nat.decode_preferred_workspace_bytes(1, 2, 32, 28, 4, 128, 1, 2048, 128) == 4 * (8 + 1) * slot
+    assert nat.decode_preferred_workspace_bytes(8, 2, 32, 28, 4, 128, 1, 8064, 128) == 768 * slot
+    for args in ((224, 2, 32, 28, 4, 128, 1, 8064, 128), (1, 2, 32, 28, 4, 64, 1, 1024, 0), (1, 4, 64, 28, 4, 128, 1, 0, 9)):
+        assert nat.decode_preferred_workspace_bytes(*args) == nat.decode_workspace_bytes(*args)
+    with pytest.raises(ValueError):
+        nat.decode_preferred_workspace_bytes(-1, 2, 32, 28, 4, 128, 1, 64, 0)
+
+
 def test_editing_validation():
     item = nat.KiviItem()
     item.quantized_tokens = 64

@@ -192,6 +192,34 @@ def test_decode_query_rows_around_the_fold(device, hq, hkv, lq):
         check_summary(out, lse, seg, q, what=f"Hq {hq} Hkv {hkv} Lq {lq} T {tokens}")
 
 
+@pytest.mark.parametrize("bits,group,tokens,heads", [(2, 32, 255 + 32, 4), (2, 64, 256 + 64, 4), (2, 32, 2100, 2),
+                                                     (4, 64, 1999, 4), (2, 32, 33000, 1), (4, 128, 9000, 8)])
+def test_decode_split_sizes_by_workspace(device, bits, group, tokens, heads):
+    # a small launch splits its segments finer when the workspace allows it
+    # (uc_kivi_decode_preferred_workspace_bytes) and keeps 8 super-tiles per
+    # split with the least workspace: both against the oracle, from one
+    # super-tile (and one token more) to 129 of them on one KV head
+    import ctypes
+
+    cache, seg = _pair(tokens, 150, bits, group, 100, device, heads=heads)
+    q = queries(1, heads=7 * heads, seed=151)
+    qd = q.to(device)
+    args = (bits, group, 7 * heads, heads, 128, 1)
+    tr = cache.residual_tokens
+    sizes = [f(1, *args, cache.quantized_tokens, tr)
+             for f in (nat.decode_workspace_bytes, nat.decode_preferred_workspace_bytes)]
+    assert sizes[1] >= sizes[0]
+    for nbytes in sizes:
+        out, lse = torch.empty_like(qd), torch.empty((7 * heads, 1), dtype=torch.float32, device=device)
+        item = cache.native_item(qd.data_ptr(), out.data_ptr(), lse.data_ptr(),
+                                 residual_key_ptr=cache.residual_key.data_ptr(),
+                                 residual_value_ptr=cache.residual_value.data_ptr(), residual_tokens=tr)
+        ws = nat.workspace(device, nbytes)
+        nat.call("uc_kivi_attn_decode", ctypes.byref(item), *args, nat.UC_BF16, nat.UC_BF16, nat.UC_BF16,
+                 1.0 / math.sqrt(128), ws.data_ptr(), nbytes, nat.stream(device))
+        check_summary(out, lse, seg, q, what=f"{nbytes} bytes of workspace")
+
+
 def test_decode_is_deterministic(device):
     cache, _ = _pair(4096, 11, 2, 32, 128, device)
     q = queries(1, seed=2).to(device)

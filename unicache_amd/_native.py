@@ -194,6 +194,7 @@ _SIGNATURES = {
     ),
     "uc_workspace_bytes": (_L, [_I, _L, _L, _L, _L, _L]),
     "uc_kivi_decode_workspace_bytes": (_L, [_L, _I, _I, _L, _L, _L, _L, _L, _L]),
+    "uc_kivi_decode_preferred_workspace_bytes": (_L, [_L, _I, _I, _L, _L, _L, _L, _L, _L]),
 }
 
 _lock = threading.Lock()
@@ -314,6 +315,18 @@ def decode_workspace_bytes(n_items, bits, group_size, heads_q, heads_kv, head_di
                                                     query_len, max_tq, max_tr))
     if size < 0:
         raise ValueError("uc_kivi_decode_workspace_bytes: bad arguments")
+    return size
+
+
+@functools.lru_cache(maxsize=256)
+def decode_preferred_workspace_bytes(n_items, bits, group_size, heads_q, heads_kv, head_dim, query_len, max_tq,
+                                     max_tr) -> int:
+    """The decode workspace with which small launches are free to split finer."""
+
+    size = int(lib().uc_kivi_decode_preferred_workspace_bytes(n_items, bits, group_size, heads_q, heads_kv, head_dim,
+                                                              query_len, max_tq, max_tr))
+    if size < 0:
+        raise ValueError("uc_kivi_decode_preferred_workspace_bytes: bad arguments")
     return size
 
 

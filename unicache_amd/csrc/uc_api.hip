@@ -80,3 +80,15 @@ extern "C" int64_t uc_kivi_decode_workspace_bytes(int64_t n_items, int bits, int
                          uc::ceil_div(max_residual_tokens, uc::kDecodeSplitTokens);
   return n_items * heads_q * query_len * splits * (head_dim + 2) * int64_t(sizeof(float));
 }
+
+extern "C" int64_t uc_kivi_decode_preferred_workspace_bytes(int64_t n_items, int bits, int group_size,
+                                                            int64_t heads_q, int64_t heads_kv, int64_t head_dim,
+                                                            int64_t query_len, int64_t max_quantized_tokens,
+                                                            int64_t max_residual_tokens) {
+  const int64_t least = uc_kivi_decode_workspace_bytes(n_items, bits, group_size, heads_q, heads_kv, head_dim,
+                                                       query_len, max_quantized_tokens, max_residual_tokens);
+  if (least < 0 || !uc::decode_mfma_supported(bits, group_size, head_dim, (heads_q / heads_kv) * query_len))
+    return least;
+  return uc::decode_mfma_preferred_workspace_bytes(n_items, heads_kv, bits, max_quantized_tokens,
+                                                   max_residual_tokens);
+}

@@ -746,5 +746,5 @@ extern "C" int uc_kivi_attn_decode_static(const uc_kivi_item *item_host, int bit
   if (rc != UC_OK) return rc;
   return decode_common(nullptr, item_host, 1, bits, group_size, heads_q, heads_kv, head_dim, query_len, q_dtype,
                        res_dtype, out_dtype, sm_scale, item_host->quantized_tokens, item_host->residual_tokens, ws,
-                       kDecodeScratchBytes, as_stream(stream), "uc_kivi_attn_decode_static");
+                       need, as_stream(stream), "uc_kivi_attn_decode_static");
 }

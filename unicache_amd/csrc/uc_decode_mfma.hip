@@ -56,6 +56,7 @@ constexpr int kResWaveTokensShort = 32, kResWaveTokensLong = 64;
 inline int64_t res_wave_tokens(int64_t max_tr) {
   return max_tr <= kWaves * kResWaveTokensShort ? kResWaveTokensShort : kResWaveTokensLong;
 }
+constexpr int64_t kCus = 256;       // CUs of an MI355X
 constexpr int kWgPerCu = 3;         // resident workgroups per CU (LDS: ~51 KB each; <= 168 VGPRs)
 constexpr float kLazyLog2 = 8.0f;   // softmax reference slack (log2 units)
 
@@ -969,7 +970,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
 // part owns channels 8c .. 8c + 7 of one query row, so a row's 16 threads read
 // each partial row as one contiguous 256-byte run; a part has only the threads
 // of the query rows (rounded to whole waves).  The splits are dealt to
-// `parts` (1, 2 or 4) parts of the block in contiguous runs; a part takes its
+// `parts` (1, 2, 4 or 8) parts of the block in contiguous runs; a part takes its
 // run in rounds of kCombineRound, every load of a round issued before any
 // arithmetic, with an online (M, L): a round that raises the maximum rescales
 // the sums first.  The parts then merge through LDS, part 0 writes the output
@@ -1097,6 +1098,16 @@ int64_t decode_mfma_num_splits(int bits, int64_t nst, int64_t max_tq, int64_t ma
   return ceil_div(max_tq, decode_mfma_split_tokens(bits, nst)) + ceil_div(max_tr, decode_mfma_res_split_tokens(max_tr));
 }
 
+int64_t decode_mfma_preferred_workspace_bytes(int64_t n_items, int64_t heads_kv, int bits, int64_t max_tq,
+                                              int64_t max_tr) {
+  const int64_t units = n_items * heads_kv;
+  const int64_t least = decode_mfma_workspace_bytes(n_items, heads_kv,
+                                                    decode_mfma_num_splits(bits, kDecodeMfmaNst, max_tq, max_tr));
+  // finer splits (choose_super_tiles) stay within one round of workgroup slots
+  const int64_t fine = min(units * decode_mfma_num_splits(bits, 1, max_tq, max_tr), kWgPerCu * kCus);
+  return max(least, decode_mfma_workspace_bytes(1, 1, fine));
+}
+
 bool decode_mfma_supported(int bits, int group, int64_t D, int64_t rows) {
   return (bits == 2 || bits == 4) && (group == 32 || group == 64 || group == 128) && D == kD && rows <= 16;
 }
@@ -1141,24 +1152,48 @@ static void launch_group(bool table, int rd, dim3 grid, hipStream_t stream, cons
     launch_typed<BITS, G, UC_BF16>(table, grid, stream, items_dev, one, p);
 }
 
+// Super-tiles per packed split of a launch.  `nst` per split is the right size
+// for launches of several rounds of workgroup slots (kWgPerCu per CU): there a
+// split's fixed cost counts.  A launch that does not fill one round is bound by
+// the longest split's serial chain instead, so it takes the split size with the
+// least estimated time: the chain's super-tiles at the measured 1.36, 1.8 or
+// 2.7 us each with 1, 2 or 3 workgroups on a CU (alone, a wave leaves half its
+// SIMD's issue slots idle; three waves fill them), plus 0.09 us per split that
+// the combine reads, in units of 0.09 us.  Measured, call to call: 8 sequences
+// of 2048 tokens at 2 bits 21.0 -> 12.6 us (1 super-tile), 8 x 8192 21.7 ->
+// 18.1 us (3), one 32768-token segment 21.9 -> 16.2 us (3; 18.6 with 2, 17.2
+// with 4), 8 x 8192 at 4 bits 21.8 -> 18.2 us (3); the estimate picked the
+// fastest or within 0.2 us of it on 15 shapes of 8 to 1024 super-tiles a unit.
+// `workspace_bytes` caps the choice: callers may bring the least workspace.
+static int64_t choose_super_tiles(int64_t nst, int64_t n_items, int64_t Hkv, int bits, int64_t max_tq, int64_t max_tr,
+                                  int64_t segs, int64_t workspace_bytes) {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return nst;
+  const int64_t units = n_items * Hkv, round = kWgPerCu * int64_t(cus);
+  const auto splits = [&](int64_t n) { return decode_mfma_num_splits(bits, n, max_tq, max_tr); };
+  // Twice the super-tiles when that fits the launch into one round and `nst`
+  // does not: a batch-1 32k context over 28 layers then runs as one full round
+  // instead of ~1.9 (+3 % measured).
+  if (units * splits(nst) > round) return units * splits(2 * nst) <= round ? 2 * nst : nst;
+  const int64_t n_super = ceil_div(max_tq, decode_mfma_split_tokens(bits, 1));
+  int64_t best = nst, best_cost = INT64_MAX;
+  for (int64_t n = nst; n >= 1; --n) {
+    const int64_t sp = ceil_div(n_super, n), groups = units * splits(n);
+    if (sp == 0 || groups > round || decode_mfma_workspace_bytes(n_items, Hkv, splits(n)) > workspace_bytes) break;
+    const int64_t tile = groups <= cus ? 15 : groups <= 2 * cus ? 20 : 30;
+    const int64_t cost = ceil_div(n_super, sp) * tile + segs * splits(n);
+    if (cost < best_cost) best = n, best_cost = cost;
+  }
+  return best;
+}
+
 int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single, int64_t n_items, int bits,
                        int group_size, int64_t Hq, int64_t Hkv, int64_t Lq, int q_dtype, int res_dtype,
                        int out_dtype, float sm_scale, int64_t max_tq, int64_t max_tr, int64_t nst, int64_t segs,
                        void *workspace, int64_t workspace_bytes, hipStream_t stream) {
-  // Twice the super-tiles per split when that fits the launch into one round of
-  // workgroup slots (kWgPerCu per CU) and `nst` does not: a batch-1 32k context then
-  // runs as one full round instead of ~1.9 (+3 % measured).  Fewer splits, so
-  // the workspace sized for `nst` still fits.
-  {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0) {
-      const int64_t units = n_items * Hkv, round = kWgPerCu * int64_t(cus);
-      if (units * decode_mfma_num_splits(bits, nst, max_tq, max_tr) > round &&
-          units * decode_mfma_num_splits(bits, 2 * nst, max_tq, max_tr) <= round)
-        nst *= 2;
-    }
-  }
+  nst = choose_super_tiles(nst, n_items, Hkv, bits, max_tq, max_tr, segs, workspace_bytes);
   const int64_t s_tok = decode_mfma_split_tokens(bits, nst);
   MfmaParams p{};
   p.Hq = Hq; p.Hkv = Hkv; p.Lq = Lq; p.group = Hq / Hkv; p.rows = p.group * Lq;
@@ -1205,12 +1240,14 @@ int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single
   if (rc != UC_OK) return rc;
   UC_REQUIRE(segs >= 1 && n_items % segs == 0, "decode: %lld items do not form groups of %lld segments",
              (long long)n_items, (long long)segs);
-  // one block per (query group, KV head): `parts` runs of about 12 splits each
-  // (at most 4), each part with the threads of the query rows
-  const int64_t nflat = segs * p.splits_total;
-  const int parts = nflat > 36 ? 4 : nflat > 12 ? 2 : 1;
+  // one block per (query group, KV head): enough parts that each takes its run
+  // of splits in one round of loads, as far as the block's threads go (a run of
+  // two rounds cost the 33 splits of a 32k segment 0.7 us of 17.9)
+  const int64_t nflat = segs * p.splits_total, span = ceil_div(p.rows * 16, int64_t(kWave)) * kWave;
+  int parts = 1;
+  while (nflat > kCombineRound * parts && 2 * parts * span <= kCombineMaxThreads) parts *= 2;
   const dim3 cgrid(static_cast<unsigned>(n_items / segs), static_cast<unsigned>(Hkv));
-  const dim3 cblock(static_cast<unsigned>(parts * ceil_div(p.rows * 16, int64_t(kWave)) * kWave));
+  const dim3 cblock(static_cast<unsigned>(parts * span));
   const size_t lds = size_t(cblock.x / parts) * (parts - 1) * 10 * sizeof(float);
   if (table)
     hipLaunchKernelGGL((decode_mfma_combine<true>), cgrid, cblock, lds, stream, items_dev, one, p, parts);

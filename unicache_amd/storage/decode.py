@@ -126,8 +126,8 @@ class KiviDecodeBatch:
         self.table = torch.frombuffer(bytearray(raw), dtype=torch.uint8).to(self.device)
         self.max_tq = max(c.quantized_tokens for c in caches)
         self.max_tr = max(c.residual_tokens for c in caches)
-        self.ws_bytes = nat.decode_workspace_bytes(len(caches), first.k_bits, first.group_size, hq,
-                                                   first.num_kv_heads, d, lq, self.max_tq, self.max_tr)
+        self.ws_bytes = nat.decode_preferred_workspace_bytes(len(caches), first.k_bits, first.group_size, hq,
+                                                             first.num_kv_heads, d, lq, self.max_tq, self.max_tr)
         if self.workspace is None or self.workspace.numel() < self.ws_bytes:
             self.workspace = nat.workspace(self.device, self.ws_bytes)
         self._guard = _TableGuard(caches, tensors)
@@ -279,8 +279,8 @@ class MixedDecodeBatch:
         self.n_items, self.max_tq, self.max_tr = n, max_tq, max_tr
         lq, hq, d = self.shape
         # sized for the longest window the reserve allows, so appends keep it
-        self.ws_bytes = nat.decode_workspace_bytes(n, self.bits, self.group_size, hq, self.kv_heads, d, lq,
-                                                   max_tq + self._room, max_tr + self._room)
+        self.ws_bytes = nat.decode_preferred_workspace_bytes(n, self.bits, self.group_size, hq, self.kv_heads, d, lq,
+                                                             max_tq + self._room, max_tr + self._room)
         if getattr(self, "workspace", None) is None or self.workspace.numel() < self.ws_bytes:
             self.workspace = nat.workspace(self.device, self.ws_bytes)
         self._streams = [streams[id(c)] for c in caches if id(c) in streams]

@@ -102,8 +102,8 @@ def _decode_summary(cache: "PackedKIVICache", query: torch.Tensor, *, include_re
     item = cache.native_item(q.data_ptr(), out.data_ptr(), lse.data_ptr(),
                              residual_key_ptr=nat.ptr(cache.residual_key) if tr else None,
                              residual_value_ptr=nat.ptr(cache.residual_value) if tr else None, residual_tokens=tr)
-    ws_bytes = nat.decode_workspace_bytes(1, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d, lq,
-                                          cache.quantized_tokens, tr)
+    ws_bytes = nat.decode_preferred_workspace_bytes(1, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d, lq,
+                                                    cache.quantized_tokens, tr)
     ws = nat.workspace(device, ws_bytes)
     res_dtype = cache.residual_key.dtype if tr else q.dtype
     nat.call(
@@ -205,8 +205,8 @@ def packed_summary_with_dense(
                              residual_value_ptr=dv.data_ptr() if tr else None, residual_tokens=tr)
     res_code = nat.dtype_code(dk.dtype if tr else q.dtype)
     if lq <= _max_decode_query_len(cache, hq):
-        ws_bytes = nat.decode_workspace_bytes(1, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d, lq,
-                                              cache.quantized_tokens, tr)
+        ws_bytes = nat.decode_preferred_workspace_bytes(1, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d,
+                                                        lq, cache.quantized_tokens, tr)
         entry = "uc_kivi_attn_decode"
     else:
         if d != 128 or cache.group_size not in (32, 64, 128) or (tr and dk.dtype not in (torch.bfloat16,
@@ -490,7 +490,7 @@ def decode_segments_summary(packed: list, query: torch.Tensor, dense: list) -> t
         items[j] = nat.KiviItem(None, None, None, None, None, None, key.data_ptr(), value.data_ptr(), q.data_ptr(),
                                 out.data_ptr(), lse.data_ptr(), 0, t, 0, key.stride(0), key.stride(1))
         max_tr = max(max_tr, t)
-    ws_bytes = nat.decode_workspace_bytes(n, first.k_bits, first.group_size, hq, hkv, d, lq, max_tq, max_tr)
+    ws_bytes = nat.decode_preferred_workspace_bytes(n, first.k_bits, first.group_size, hq, hkv, d, lq, max_tq, max_tr)
     workspace = nat.workspace(device, ws_bytes)
     nat.call("uc_kivi_attn_decode_segments_host", items, n, first.k_bits, first.group_size, hq, hkv, d, lq,
              nat.dtype_code(q.dtype), nat.dtype_code(res_dtype), nat.dtype_code(q.dtype), 1.0 / math.sqrt(d),
@@ -629,7 +629,7 @@ def dense_attention_summary(
                         out.data_ptr(), lse.data_ptr(), 0, tokens, 0)
     bits, group = 2, 32  # no packed tokens: only the dense (residual) part is read
     if lq <= max(1, 16 // (hq // hkv)):
-        ws_bytes = nat.decode_workspace_bytes(1, bits, group, hq, hkv, d, lq, 0, tokens)
+        ws_bytes = nat.decode_preferred_workspace_bytes(1, bits, group, hq, hkv, d, lq, 0, tokens)
         entry = "uc_kivi_attn_decode"
     else:
         if d != 128:

@@ -381,6 +381,50 @@ def test_mq_ragged_tiles_and_rows(device, bits, group, tokens, residual, lq):
     check_summary(out, lse, seg, q, what=f"mq G{group} T{tokens} Lq{lq}")
 
 
+@pytest.mark.parametrize("lq,tokens,dense,qdtype", [(1171, 128 + 100, 1, torch.bfloat16), (1180, 700, 65, torch.float16),
+                                                    (2345, 64, 300, torch.bfloat16), (3520, 200, 0, torch.bfloat16)])
+def test_mq_workgroups_of_one_and_two_halves(device, lq, tokens, dense, qdtype):
+    # 28/4 heads: 260 work items (4-wave workgroups: every tile in one half),
+    # 516 (8 waves, two halves) and 772 (4 waves again), over 1 to 12 key tiles
+    # that end inside a tile, all or none of them packed but one
+    from unicache_amd.storage.kivi_cuda import packed_segments_summary
+
+    cache, seg = _pair(tokens, 97, 2, 32, 37 if tokens > 100 else 0, device)
+    dk, dv = kv_pair(dense, seed=98, dtype=qdtype)
+    q = queries(lq, seed=99, dtype=qdtype)
+    out, lse = packed_segments_summary([cache], q.to(device), [(dk.to(device), dv.to(device))])
+    key, value = K.dequantize(seg, "fp32")
+    rows = np.r_[0:40, lq // 2:lq // 2 + 40, lq - 40:lq]  # the oracle on a few rows of the first and last blocks
+    eo, el = A.attention_summary(f32(q)[rows], np.concatenate([key, f32(dk)]), np.concatenate([value, f32(dv)]))
+    assert_close(f32(out)[rows], eo, what="out")
+    assert_close(f32(lse)[:, rows], el, max_abs=1e-2, mean_abs=1e-3, what="lse")
+    # the other rows: every query row written, rows of one query head independent of their block
+    assert torch.isfinite(out.float()).all() and torch.isfinite(lse).all()
+    part, _ = packed_segments_summary([cache], q[5:700].to(device), [(dk.to(device), dv.to(device))])
+    # (the fp32 results differ by rounding, so a bf16 output moves by one step at
+    # most: 2^-5 = 0.03125 for outputs below 8, which an average of N(0,1) values is)
+    assert float(out.abs().max()) < 8
+    assert_close(f32(part), f32(out)[5:700], max_abs=0.0313, mean_abs=5e-4, what="part of the rows")
+
+
+def test_mq_table_of_both_kinds(device):
+    # one table call whose queries take workgroups of one half and of two (two
+    # launches): each equals its own call bit for bit
+    from unicache_amd.storage.kivi_cuda import packed_segments_summary, packed_table_summaries
+
+    cache, _ = _pair(600, 100, 2, 32, 40, device)
+    entries, want = [], []
+    for i, lq in enumerate((300, 1200, 90)):
+        q = queries(lq, seed=101 + i).to(device)
+        dense = [tuple(x.to(device) for x in kv_pair(70 + i, seed=110 + i))]
+        out, lse = torch.empty_like(q), torch.empty((28, lq), dtype=torch.float32, device=device)
+        entries.append((q, out, lse, [cache], dense))
+        want.append(packed_segments_summary([cache], q, dense, dense_dtype=torch.bfloat16))
+    packed_table_summaries(entries, dense_dtype=torch.bfloat16)
+    for (_, out, lse, _, _), (o, x) in zip(entries, want):
+        assert torch.equal(out, o) and torch.equal(lse, x)
+
+
 def test_mq_fp16_inputs(device):
     key, value = kv_pair(800, seed=90, dtype=torch.float16)
     cache = PackedKIVICache.from_dense(key.to(device), value.to(device), logical_token_ids=torch.arange(800),

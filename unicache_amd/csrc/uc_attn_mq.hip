@@ -3,9 +3,13 @@
 // attention (image editing: ~1088 queries x 7 query heads per KV head), one
 // softmax over every segment of a query in one launch.
 //
-// mq_attention_kernel: one workgroup (8 waves) owns 128 query rows of one KV
-// head; waves 0-3 take half of the 64-key tiles (half of the packed tiles,
-// then part of the dense ones) and waves 4-7 the rest, 32 query rows per wave.
+// mq_attention_kernel: one workgroup owns 128 query rows of one KV head, 32 per
+// wave.  In launches that fill the chip it has 4 waves (HALVES 1) and two
+// workgroups share a CU: their barriers are their own, so the one's matrix
+// phases drift into the other's softmax.  In smaller launches it has 8 waves
+// (HALVES 2): waves 0-3 take half of the 64-key tiles (half of the packed
+// tiles, then part of the dense ones), waves 4-7 the rest, and the two merge at
+// the end (one_half has the rule and what both measured).
 // A tile's keys and values reach double-buffered LDS slots as fp16 or 16-bit
 // dense rows in one swizzled layout, one barrier per tile:
 //   packed tiles: the half's 256 threads load the tile's code words and fp16
@@ -94,8 +98,6 @@ constexpr int kXcds = 8;  // XCDs of an MI355X; launch index i runs on XCD i % 8
 constexpr int kTile = 64;  // keys per tile
 constexpr int kHalfWaves = 4;
 constexpr int kHalfThreads = kHalfWaves * kWave;
-constexpr int kAttnWaves = 2 * kHalfWaves;
-constexpr int kAttnThreads = kAttnWaves * kWave;
 constexpr int kRowsPerWave = 32;
 constexpr int kMqRows = kHalfWaves * kRowsPerWave;  // query rows per workgroup
 // The reference of a query column is raised only when a logit exceeds it by
@@ -113,16 +115,18 @@ constexpr int kSlotBytes = 2 * kTile * 256;
 constexpr int kValueBytes = kTile * 256;  // values start after the keys of a slot
 constexpr int kMergeFloats = 2 * 8 * 4 + 4;  // O^T (2 query blocks x 8 channel blocks x 4) + m[2], l[2]
 constexpr int kRowPad = kD + 8;              // output staging row, in elements
+template <int HALVES, class OutT>
 struct MqShared {
   union {
-    uint32_t slot[2][2][kSlotBytes / 4];  // [key half][buffer]: the tiles
-    struct {                              // after the last tile:
-      float mg[kHalfWaves][kMergeFloats * kWave];  // (O^T, m, l) of the second half's waves
-      uint32_t ob[kMqRows * kRowPad];              // normalised output rows (fp32 size)
+    uint32_t slot[HALVES][2][kSlotBytes / 4];  // [key half][buffer]: the tiles
+    struct {                                   // after the last tile:
+      float mg[HALVES == 2 ? kHalfWaves : 1][HALVES == 2 ? kMergeFloats * kWave : 4];  // (O^T, m, l) of half 1's waves
+      alignas(16) OutT ob[kMqRows * kRowPad];  // normalised output rows
     } ep;
   };
 };
-static_assert(sizeof(MqShared) <= 160 * 1024, "fits the LDS of a workgroup");
+static_assert(sizeof(MqShared<2, float>) <= 160 * 1024 && sizeof(MqShared<1, float>) <= 80 * 1024,
+              "one workgroup of two halves or two workgroups of one fit the LDS of a CU");
 
 // ------------------------------------------------------------ launch table --
 // Everything a launch needs travels by value in the kernel arguments: up to
@@ -656,21 +660,23 @@ __device__ __forceinline__ void convert_queries(u32x4 (&qf)[2][4]) {
 }
 
 // Work item of query Q: 128 query rows (row block rb) of KV head h over every
-// segment of the query.  Each half takes half of the packed tiles (fp16
+// segment of the query.  Of two halves each takes half of the packed tiles (fp16
 // operands) and then dense tiles (dtype RD) up to n0 = ceil(tiles / 2) for
 // the first half.
-template <int BITS, int QD, int RD, int OD>
+template <int HALVES, int BITS, int QD, int RD, int OD>
 __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQuery &Q, int64_t h, int64_t rb) {
-  __shared__ __align__(16) MqShared sh;
+  typedef typename DtypeOf<OD>::T OutT;
+  __shared__ __align__(16) MqShared<HALVES, OutT> sh;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: tile choices stay scalar
-  const int half = wave / kHalfWaves, hw = wave % kHalfWaves;
+  const int half = HALVES == 2 ? wave / kHalfWaves : 0, hw = wave % kHalfWaves;
   const int tid_h = tid - half * kHalfThreads;
   const int r = lane & 15, kap = lane >> 4;
   const int64_t row0 = rb * kMqRows + hw * kRowsPerWave;
 
-  const int n_tiles = Q.pt + Q.dt, n0 = (n_tiles + 1) / 2;
-  const int q0 = (Q.pt + 1) / 2, d0 = n0 - q0;  // the first half's packed and dense tiles
+  // the first half's tiles, and the packed and dense ones among them
+  const int n_tiles = Q.pt + Q.dt, n0 = (n_tiles + HALVES - 1) / HALVES;
+  const int q0 = (Q.pt + HALVES - 1) / HALVES, d0 = n0 - q0;
   const int pb = half ? q0 : 0, db = half ? d0 : 0;
   const int n_pre = half ? Q.pt - q0 : q0;
   const int count = n_pre + (half ? Q.dt - d0 : d0);
@@ -762,8 +768,10 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
     u32x4 *qs = reinterpret_cast<u32x4 *>(sh.slot[0][1]) + hw * 8 * kWave + lane;
     if (half == 0) {
       load_queries(qf, Q, tb, h, row0);
+      if constexpr (HALVES == 2) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) qs[j * kWave] = qf[j / 4][j % 4];
+        for (int j = 0; j < 8; ++j) qs[j * kWave] = qf[j / 4][j % 4];
+      }
     }
     if (n_pre > 0) {
       store_keys<BITS>(pr, tid_h, half_base, magic);
@@ -827,8 +835,8 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
 
   // merge: the second half hands (O^T, m, l) of its lanes to the wave with the
   // same rows in the first half
-  float *mg = sh.ep.mg[hw];
-  if (half == 1) {
+  float *mg = sh.ep.mg[HALVES == 2 ? hw : 0];
+  if (HALVES == 2 && half == 1) {
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
 #pragma unroll
@@ -839,13 +847,13 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
       mg[(66 + qb) * kWave + lane] = st.l[qb];
     }
   }
-  __syncthreads();
-  typedef typename DtypeOf<OD>::T OutT;
-  OutT *ob = reinterpret_cast<OutT *>(sh.ep.ob) + hw * kRowsPerWave * kRowPad;
+  if constexpr (HALVES == 2) __syncthreads();
+  OutT *ob = sh.ep.ob + hw * kRowsPerWave * kRowPad;
   if (half == 0) {
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      const float m2 = mg[(64 + qb) * kWave + lane], l2 = mg[(66 + qb) * kWave + lane];
+      const float m2 = HALVES == 2 ? mg[(64 + qb) * kWave + lane] : kNegInf;
+      const float l2 = HALVES == 2 ? mg[(66 + qb) * kWave + lane] : 0.0f;
       const float M = fmaxf(st.m[qb], m2);
       const float M_ref = M == kNegInf ? 0.0f : M;
       const float a1 = fast_exp2(st.m[qb] - M_ref), a2 = fast_exp2(m2 - M_ref);
@@ -855,7 +863,9 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
       for (int cb = 0; cb < 8; ++cb)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const float o = st.o[qb][cb][v] * a1 + mg[((qb * 8 + cb) * 4 + v) * kWave + lane] * a2;
+          const float o = HALVES == 2
+                              ? st.o[qb][cb][v] * a1 + mg[((qb * 8 + cb) * 4 + v) * kWave + lane] * a2
+                              : st.o[qb][cb][v];
           store_from_f32<OD>(ob, (16 * qb + r) * kRowPad + 16 * cb + 4 * kap + v, o * inv);
         }
       const int64_t row = row0 + 16 * qb + r;
@@ -866,13 +876,14 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
     }
   }
   __syncthreads();
-  {  // each half writes 16 of the 32 rows
+  {  // each half writes its share of the 32 rows
     constexpr int kChunk = 16 / sizeof(OutT);  // elements per 16-byte store
     constexpr int kPerRow = kD / kChunk;
-    const OutT *obw = reinterpret_cast<const OutT *>(sh.ep.ob) + hw * kRowsPerWave * kRowPad;
+    constexpr int kShare = kRowsPerWave / HALVES;
+    const OutT *obw = sh.ep.ob + hw * kRowsPerWave * kRowPad;
 #pragma unroll
-    for (int q = 0; q < kRowsPerWave / 2 * kPerRow / kWave; ++q) {
-      const int idx = q * kWave + lane, rr = half * (kRowsPerWave / 2) + idx / kPerRow, cc = (idx % kPerRow) * kChunk;
+    for (int q = 0; q < kShare * kPerRow / kWave; ++q) {
+      const int idx = q * kWave + lane, rr = half * kShare + idx / kPerRow, cc = (idx % kPerRow) * kChunk;
       const int64_t row = row0 + rr;
       if (row >= Q.rows) continue;
       const uint32_t gq = fast_div(static_cast<uint32_t>(row), Q.lq);
@@ -888,8 +899,8 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
 // work items x * per_xcd .. (row blocks of KV head h at h * row_blocks ..): a
 // contiguous run, mostly of one KV head, whose keys and values its own L2
 // then holds, and one eighth of every query.  Queries come longest first.
-template <int BITS, int QD, int RD, int OD>
-__global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2))) void mq_attention_kernel(
+template <int HALVES, int BITS, int QD, int RD, int OD>
+__global__ __launch_bounds__(HALVES *kHalfThreads) __attribute__((amdgpu_waves_per_eu(2))) void mq_attention_kernel(
     MqTable tb) {
   const int x = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
   int qi = 0;
@@ -897,7 +908,7 @@ __global__ __launch_bounds__(kAttnThreads) __attribute__((amdgpu_waves_per_eu(2)
   const MqQuery &Q = tb.q[qi];
   const int w = x * Q.per_xcd + (j - Q.slot0);
   if (w >= Q.row_blocks * tb.Hkv) return;  // uniform: the whole workgroup leaves
-  mq_attention_body<BITS, QD, RD, OD>(tb, Q, w / Q.row_blocks, w % Q.row_blocks);
+  mq_attention_body<HALVES, BITS, QD, RD, OD>(tb, Q, w / Q.row_blocks, w % Q.row_blocks);
 }
 
 }  // namespace
@@ -1065,6 +1076,30 @@ struct TableBuilder {
     return UC_OK;
   }
 
+  // Whether workgroups of one half (4 waves, every tile, two a CU) finish query
+  // `q` sooner than workgroups of two (8 waves, half the tiles each, one a CU).
+  // The choice looks at the query alone, so a query's result does not depend on
+  // the others of its launch.  Up to one work item per CU the one half would
+  // leave half of the chip's wave slots empty (GQA 28/4, two halves -> one: 240
+  // items over 2304 keys 49.0 -> 59.7 us); beyond, it wins (264 items over 2048
+  // keys 86.6 -> 73.9 us, 504 over 8192 290 -> 273 us, 900 over 8192 576 -> 528
+  // us), except where its second round of two items a CU is at most half full:
+  // 548 items over 8192 keys 430.7 -> 434.7 us, 768 434.6 -> 440.7 us.
+  bool one_half(const MqQuery &q) const {
+    constexpr int64_t kCus = 256;  // of an MI355X
+    const int64_t items = q.row_blocks * heads_kv;
+    return items > kCus && !(items > 2 * kCus && items <= 3 * kCus);
+  }
+
+  // Keeps the queries of one kind of workgroup; false if there are none.
+  bool keep(bool one) {
+    int n = 0;
+    for (int i = 0; i < t.n_queries; ++i)
+      if (one_half(t.q[i]) == one) t.q[n++] = t.q[i];
+    t.n_queries = n;
+    return n > 0;
+  }
+
   // Orders the queries longest first (segments stay where they are), assigns
   // the launch slots and returns the grid size.
   int64_t finish(float sm_scale) {
@@ -1085,16 +1120,26 @@ struct TableBuilder {
   }
 };
 
-int mq_launch(TableBuilder &b, int bits, int q_dtype, int res_dtype, int out_dtype, float sm_scale,
+int mq_launch(const TableBuilder &all, int bits, int q_dtype, int res_dtype, int out_dtype, float sm_scale,
               hipStream_t stream, const char *what) {
-  const int64_t grid = b.finish(sm_scale);
-  UC_REQUIRE(grid < kOffsetLimit, "%s: launch too large", what);
-  attn_config(bits, q_dtype, res_dtype, out_dtype, [&](auto bb, auto qd, auto rd, auto od) {
-    hipLaunchKernelGGL((mq_attention_kernel<decltype(bb)::value, decltype(qd)::value, decltype(rd)::value,
-                                            decltype(od)::value>),
-                       dim3(static_cast<unsigned>(grid)), dim3(kAttnThreads), 0, stream, b.t);
-  });
-  return check_launch(what);
+  for (const bool one : {true, false}) {  // one launch, or two where the queries' kinds of workgroup differ
+    TableBuilder b = all;
+    if (!b.keep(one)) continue;
+    const int64_t grid = b.finish(sm_scale);
+    UC_REQUIRE(grid < kOffsetLimit, "%s: launch too large", what);
+    attn_config(bits, q_dtype, res_dtype, out_dtype, [&](auto bb, auto qd, auto rd, auto od) {
+      constexpr int B = decltype(bb)::value, Q = decltype(qd)::value, R = decltype(rd)::value, O = decltype(od)::value;
+      if (one)
+        hipLaunchKernelGGL((mq_attention_kernel<1, B, Q, R, O>), dim3(static_cast<unsigned>(grid)),
+                           dim3(kHalfThreads), 0, stream, b.t);
+      else
+        hipLaunchKernelGGL((mq_attention_kernel<2, B, Q, R, O>), dim3(static_cast<unsigned>(grid)),
+                           dim3(2 * kHalfThreads), 0, stream, b.t);
+    });
+    const int rc = check_launch(what);
+    if (rc != UC_OK) return rc;
+  }
+  return UC_OK;
 }
 
 }  // namespace

@@ -977,6 +977,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
 // and the LSE of the group's first item.  Splits without work wrote (-inf, 0)
 // and no partial: their weight is 0 and their partial is not read.
 constexpr int kCombineRound = 16;
+constexpr int kCombineRun = 12;  // splits a part takes before the launch adds parts
 constexpr int kCombineMaxThreads = 1024;
 
 // Eight channels of output element `idx` on, from fp32 (one 16-byte store for
@@ -1241,11 +1242,11 @@ int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single
   UC_REQUIRE(segs >= 1 && n_items % segs == 0, "decode: %lld items do not form groups of %lld segments",
              (long long)n_items, (long long)segs);
   // one block per (query group, KV head): enough parts that each takes its run
-  // of splits in one round of loads, as far as the block's threads go (a run of
-  // two rounds cost the 33 splits of a 32k segment 0.7 us of 17.9)
+  // of splits in less than one round of loads, as far as the block's threads go
+  // (a run of two rounds cost the 33 splits of a 32k segment 0.7 us of 17.9)
   const int64_t nflat = segs * p.splits_total, span = ceil_div(p.rows * 16, int64_t(kWave)) * kWave;
   int parts = 1;
-  while (nflat > kCombineRound * parts && 2 * parts * span <= kCombineMaxThreads) parts *= 2;
+  while (nflat > kCombineRun * parts && 2 * parts * span <= kCombineMaxThreads) parts *= 2;
   const dim3 cgrid(static_cast<unsigned>(n_items / segs), static_cast<unsigned>(Hkv));
   const dim3 cblock(static_cast<unsigned>(parts * span));
   const size_t lds = size_t(cblock.x / parts) * (parts - 1) * 10 * sizeof(float);

@@ -254,6 +254,21 @@ def test_gqa_logits_mfma_tiles(device, lq, tokens, dtype):
     assert torch.equal(gqa_query_key_logits(q.to(device), kh), got)
 
 
+# Waves with all of their 64 rows (whole-line stores), with some of them and
+# with none; one tile a workgroup and several; a last tile that is not full;
+# rows that do and do not start on 16 bytes.
+@pytest.mark.parametrize("lq,tokens,dtype", [(64, 64, torch.bfloat16), (10, 132, torch.bfloat16), (37, 192, torch.float16),
+                                             (128, 191, torch.bfloat16), (97, 4096, torch.bfloat16),
+                                             (130, 8196, torch.float16)])
+def test_gqa_logits_store_paths(device, lq, tokens, dtype):
+    key, _ = kv_pair(tokens, seed=33, dtype=dtype)
+    q = queries(lq, seed=34, dtype=dtype)
+    got = f32(gqa_query_key_logits(q.to(device), key.to(device)))
+    # exact products, 128 additions in fp32 each way, and the same again for the oracle
+    bound = 2 * 130 * 2.0 ** -24 * A.gqa_logits(np.abs(f32(q)), np.abs(f32(key)))
+    assert (np.abs(got - A.gqa_logits(f32(q), f32(key))) <= bound).all()
+
+
 @pytest.mark.parametrize("pdtype,vdtype", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.bfloat16),
                                            (torch.float32, torch.float16)])
 def test_gqa_pv_mfma_tiles(device, pdtype, vdtype):

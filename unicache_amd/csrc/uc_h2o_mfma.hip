@@ -107,6 +107,9 @@ struct HsShared {
   float col[2][kHsWaves][kHsTile];
 };
 
+// s_waitcnt immediate (gfx9 layout): vmcnt <= n (6 bits), expcnt and lgkmcnt not waited on
+constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
+
 // The key rows [t_begin, t_end) of one KV head, streamed a tile at a time.
 // Rows past t_end fall outside the buffer resource and read as zero.
 struct KeyStream {
@@ -153,8 +156,34 @@ struct KeyStream {
     if (i + kHsStages - 1 < n_tiles) issue(sh, i + kHsStages - 1);
   }
 
-  // s_waitcnt immediates (gfx9 layout): vmcnt <= N, expcnt and lgkmcnt not waited on
-  static constexpr int kWaitVm0 = 0x0F70, kWaitVm4 = 0x0F74, kWaitVm8 = 0x0F78;
+  // acquire() of a loop whose every tile before this one ended with exactly 16
+  // stores by this thread's wave.  Stores and loads share one in-order counter:
+  // a wait that counted the loads alone would also wait for the stores of the
+  // tiles before.  Issued after the loads of tile i: the stores of the last two
+  // tiles and the loads of tile i + 1.
+  __device__ __forceinline__ void acquire_past_stores(HsShared &sh, int i) const {
+    static_assert(kHsStages == 3, "the counts below");
+    const bool ahead = i + 1 < n_tiles;
+    if (i >= 2) {
+      if (ahead)
+        __builtin_amdgcn_s_waitcnt(wait_vm(4 + 32));
+      else
+        __builtin_amdgcn_s_waitcnt(wait_vm(32));
+    } else if (i == 1) {
+      if (ahead)
+        __builtin_amdgcn_s_waitcnt(wait_vm(4 + 16));
+      else
+        __builtin_amdgcn_s_waitcnt(wait_vm(16));
+    } else if (ahead) {
+      __builtin_amdgcn_s_waitcnt(wait_vm(4));
+    } else {
+      __builtin_amdgcn_s_waitcnt(wait_vm(0));
+    }
+    __syncthreads();
+    if (i + kHsStages - 1 < n_tiles) issue(sh, i + kHsStages - 1);
+  }
+
+  static constexpr int kWaitVm0 = wait_vm(0), kWaitVm4 = wait_vm(4), kWaitVm8 = wait_vm(8);
 };
 
 template <int DT>
@@ -355,10 +384,25 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3)))
   }
 }
 
+// x, with the 4-lane quads of every 16 lanes that MASK names taken from `from`
+// of the lane a row rotation (DPP control ROR) away.
+template <int ROR, int MASK>
+__device__ __forceinline__ float from_lane_quads(float x, float from) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(from), ROR, 0xF, MASK, false));
+}
+
 // Logits of dense keys, fp32 [Hq][Lq][T] = scale * q . k (physical.py:20-39).
 // The tiles are computed as S^T = K Q^T, so lane (n, k) holds four
-// consecutive keys 16 tb + 4k .. + 3 of row 16 qb + n and writes them with one
-// 16-byte store: a store instruction covers 16 rows x 64 contiguous bytes.
+// consecutive keys 16 tb + 4k .. + 3 of row 16 qb + n.
+//
+// Bound by its stores.  Written from there, a store instruction covers 16 rows
+// x 64 bytes, half a cache line each.  Two key blocks are therefore exchanged
+// between rows n and n ^ 8 first (one DPP move a value), and a store covers 8
+// rows x 128 bytes; the waits for the key tiles leave the stores in flight.
+// 235 MB of logits (28 heads x 512 rows x 4096 keys): 57.9 us with half lines,
+// 49.0 with whole lines, 47.4 with those waits (a fill of the size: 34).  Four
+// blocks a store (4 rows x 256 bytes) need 20 registers too many: 64 us.
+// Non-temporal stores: 81 us of half lines, 55 of whole ones.
 template <int DT>
 __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3))) void qk_logits_kernel(HsParams p) {
   __shared__ __align__(16) HsShared sh;
@@ -388,10 +432,52 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3)))
     const uint32_t i = static_cast<uint32_t>(row) - g * lq;
     ro[qb] = row < p.rows ? ((h * p.group + g) * p.Lq + i) * p.T : -1;
   }
+  // every row of the wave exists and rows take whole stores: full tiles end with
+  // exactly 16 stores, which acquire_past_stores counts on
+  const bool whole = vec && row0 + kHsRowsPerWave <= p.rows;
+  // where this lane's first store of a block pair goes: row n & 7 of 16 qb,
+  // keys 4k .. + 3 of the pair's first (n < 8) or second block; its other store
+  // is 8 rows on (rows are contiguous: [Hq][Lq] of one KV head)
+  int64_t pr[kHsQB];
+#pragma unroll
+  for (int qb = 0; qb < kHsQB; ++qb) pr[qb] = ro[qb] - (r & 8) * p.T + 4 * kap + 2 * (r & 8);
   for (int i = 0; i < ks.n_tiles; ++i) {
-    ks.acquire(sh, i);
+    if (whole)
+      ks.acquire_past_stores(sh, i);
+    else
+      ks.acquire(sh, i);
     const int64_t t0 = t_begin + int64_t(i) * kHsTile;
     const uint4 *kt = sh.kt[i % kHsStages];
+    if (whole && t0 + kHsTile <= t_end) {
+      for (int tb = 0; tb < 4; tb += 2) {
+        typename HsOp<DT>::V kf[2][4];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int kb = 0; kb < 4; ++kb) kf[u][kb] = key_frag<DT>(kt, 16 * (tb + u) + r, 4 * kb + kap);
+#pragma unroll
+        for (int qb = 0; qb < kHsQB; ++qb) {
+          f4 s0 = f4{0, 0, 0, 0}, s1 = s0;
+#pragma unroll
+          for (int kb = 0; kb < 4; ++kb) {
+            s0 = HsOp<DT>::mma(kf[0][kb], qf[qb][kb], s0);
+            s1 = HsOp<DT>::mma(kf[1][kb], qf[qb][kb], s1);
+          }
+          s0 = s0 * p.scale;
+          s1 = s1 * p.scale;
+          f4 lo, hi;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            lo[v] = from_lane_quads<0x128, 0xC>(s0[v], s1[v]);
+            hi[v] = from_lane_quads<0x128, 0x3>(s1[v], s0[v]);
+          }
+          float *dst = p.logits + pr[qb] + t0 + 16 * tb;
+          *reinterpret_cast<f4 *>(dst) = lo;
+          *reinterpret_cast<f4 *>(dst + 8 * p.T) = hi;
+        }
+      }
+      continue;
+    }
 #pragma unroll
     for (int tb = 0; tb < 4; ++tb) {
       typename HsOp<DT>::V kf[4];

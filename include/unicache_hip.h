@@ -115,6 +115,24 @@ int uc_kivi_dequant(const void *key_code, int64_t kc_sh, int64_t kc_sd, int64_t 
                     uc_stream_t stream);
 
 /*
+ * uc_kivi_dequant of both tensors, and the dense rows that follow the packed
+ * ones: res_key / res_value, compact [res_rows, heads, head_dim] of
+ * `out_dtype`, are copied to the output rows after the last restored token
+ * (the whole of PackedKIVICache.dequantize, physical.py:379-423, in one launch
+ * where both parts move in 16-byte units).  res_rows may be 0.
+ */
+int uc_kivi_restore(const void *key_code, int64_t kc_sh, int64_t kc_sd, int64_t kc_sw,
+                    const void *key_scale, const void *key_min, int64_t ks_sh, int64_t ks_sd, int64_t ks_sg,
+                    const void *value_code, int64_t vc_sh, int64_t vc_st, int64_t vc_sw,
+                    const void *value_scale, const void *value_min, int64_t vs_sh, int64_t vs_st, int64_t vs_sg,
+                    int stats_dtype, int64_t heads, int64_t head_dim,
+                    int k_bits, int v_bits, int group_size, int64_t start, int64_t stop,
+                    void *out_key, void *out_value, int out_dtype,
+                    int64_t o_st, int64_t o_sh, int64_t o_sd, int64_t output_offset,
+                    const void *res_key, const void *res_value, int64_t res_rows,
+                    uc_stream_t stream);
+
+/*
  * KIVI fake quantization (quantize then dequantize, no packing) of a dense
  * [tokens, heads, head_dim] tensor, grouped along `dim` (0 = tokens for keys,
  * 2 = channels for values), written to `out` (same strides as the input).

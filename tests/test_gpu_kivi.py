@@ -460,3 +460,31 @@ def test_non_finite_inputs_match_oracle(device, native):
         fv = K.fake_quant(f32(value), bits=2, dim=-1, group_size=32)
     assert np.array_equal(f32(kivi_fake_quant_key(key.to(device), bits=2, group_size=32)), fk, equal_nan=True)
     assert np.array_equal(f32(kivi_fake_quant_value(value.to(device), bits=2, group_size=32)), fv, equal_nan=True)
+
+
+# The dense rows after the packed ones: in the packed rows' launch (16-byte
+# units), in one of their own (unaligned rows; 8 bits; other layouts), by a copy
+# (rows that are not compact or not of the wanted type).
+@pytest.mark.parametrize("bits,dtype", [(2, torch.bfloat16), (4, torch.float16), (4, torch.float32), (8, torch.bfloat16)])
+@pytest.mark.parametrize("rows,form", [(1, "compact"), (33, "compact"), (129, "shifted"), (40, "strided"), (7, "float32")])
+def test_dequantize_residual_rows(device, bits, dtype, rows, form):
+    key, value = kv_pair(192 + rows, seed=60 + rows, dtype=dtype)
+    for backend in ("cuda", "reference"):
+        cache = PackedKIVICache.from_dense(
+            key.to(device), value.to(device), logical_token_ids=torch.arange(192 + rows), token_type_id=0, k_bits=bits,
+            v_bits=bits, group_size=64, residual_length=rows, backend=backend if bits != 8 else "reference")
+        assert cache.quantized_tokens == 192
+        dense = [cache.residual_key, cache.residual_value]
+        if form == "shifted":  # rows that start one element past a 16-byte boundary
+            dense = [torch.cat([x.reshape(-1)[:1], x.reshape(-1)])[1:].view_as(x) for x in dense]
+        elif form == "strided":
+            dense = [x.transpose(0, 1).contiguous().transpose(0, 1) for x in dense]
+        elif form == "float32":
+            dense = [x.float() for x in dense]
+        cache.residual_key, cache.residual_value = dense
+        got = cache.dequantize(dtype)
+        for out, x, src in zip(got, dense, (key, value)):
+            assert out.dtype == dtype and torch.equal(out[192:].cpu(), src[192:])
+        rk, rv = torch.empty_like(got[0][:192]), torch.empty_like(got[1][:192])
+        cache.dequantize_into(rk, rv, start=0, stop=192, output_offset=0)
+        assert torch.equal(got[0][:192], rk) and torch.equal(got[1][:192], rv)

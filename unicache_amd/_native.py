@@ -117,6 +117,12 @@ _SIGNATURES = {
          _P, _L, _L, _L, _P, _P, _L, _L, _L,
          _I, _L, _L, _I, _I, _I, _L, _L, _P, _P, _I, _L, _L, _L, _L, _P],
     ),
+    "uc_kivi_restore": (
+        _I,
+        [_P, _L, _L, _L, _P, _P, _L, _L, _L,
+         _P, _L, _L, _L, _P, _P, _L, _L, _L,
+         _I, _L, _L, _I, _I, _I, _L, _L, _P, _P, _I, _L, _L, _L, _L, _P, _P, _L, _P],
+    ),
     "uc_kivi_fake_quant": (_I, [_P, _L, _L, _L, _I, _L, _L, _L, _I, _I, _I, _P, _P]),
     "uc_kivi_qk": (
         _I,

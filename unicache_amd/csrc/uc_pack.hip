@@ -729,7 +729,30 @@ struct DequantArgs {
   int lg;         // log2(group_size) (tuned group sizes)
   int64_t group;  // group_size (any)
   int sd, od;     // stats and output dtype codes
+  const void *res_key, *res_value;  // dense rows that follow the packed ones, compact, of the output dtype
+  int64_t res_rows;
 };
+
+// The dense rows of a tensor into the output rows after the packed ones, one
+// unit of sizeof(T) bytes a thread; units = head_dim * element bytes / sizeof(T).
+template <typename T>
+__device__ __forceinline__ void copy_residual(const DequantArgs &a, int64_t per_tensor, uint32_t units, int elem_bytes,
+                                              int64_t idx) {
+  if (idx >= 2 * per_tensor) return;
+  const bool value = idx >= per_tensor;
+  const uint32_t i = static_cast<uint32_t>(value ? idx - per_tensor : idx);
+  const uint32_t q = i / units, u = i - q * units, heads = static_cast<uint32_t>(a.heads);
+  const uint32_t n = q / heads, h = q - n * heads;
+  const int64_t ch = int64_t(u) * (sizeof(T) / elem_bytes);
+  char *out = static_cast<char *>(value ? a.out_value : a.out_key);
+  *reinterpret_cast<T *>(out + ((a.offset + a.count + n) * a.o_st + h * a.o_sh + ch * a.o_sd) * elem_bytes) =
+      static_cast<const T *>(value ? a.res_value : a.res_key)[i];
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void copy_residual_kernel(DequantArgs a, int64_t per_tensor) {
+  copy_residual<T>(a, per_tensor, static_cast<uint32_t>(a.head_dim), sizeof(T), int64_t(blockIdx.x) * 256 + threadIdx.x);
+}
 
 // One thread per output element (token, head, channel); keys and values are
 // restored by separate halves of the grid.
@@ -952,15 +975,20 @@ __global__ __launch_bounds__(256) void dequant_value_native_kernel(DequantArgs a
   dequant_value_native_block<BITS, OD, VEC>(a, blockIdx.x);
 }
 
-// Keys (the first key_blocks workgroups, octet form) and values of equal bits
-// in one launch.
+// Keys (the first key_blocks workgroups, octet form), values of equal bits and
+// the dense rows that follow (the last workgroups, 16 bytes a thread) in one
+// launch.
 template <int BITS, int OD, int SD, bool VEC>
-__global__ __launch_bounds__(256) void dequant_kv_kernel(DequantArgs a, int64_t runs, int64_t key_blocks) {
+__global__ __launch_bounds__(256) void dequant_kv_kernel(DequantArgs a, int64_t runs, int64_t key_blocks,
+                                                         int64_t value_blocks) {
   const int64_t b = blockIdx.x;
   if (b < key_blocks)
     dequant_key_octet_block<BITS, OD, SD>(a, runs, b);
-  else
+  else if (b < key_blocks + value_blocks)
     dequant_value_native_block<BITS, OD, VEC>(a, b - key_blocks);
+  else
+    copy_residual<uint4>(a, a.res_rows * a.heads * a.head_dim / 8, static_cast<uint32_t>(a.head_dim / 8), 2,
+                         (b - key_blocks - value_blocks) * 256 + threadIdx.x);
 }
 
 // ----------------------------------------------------------- fake quant --
@@ -1299,15 +1327,19 @@ extern "C" int uc_kivi_pack(const void *key, int64_t k_st, int64_t k_sh, int64_t
   return check_launch("uc_kivi_pack");
 }
 
-extern "C" int uc_kivi_dequant(const void *key_code, int64_t kc_sh, int64_t kc_sd, int64_t kc_sw,
-                               const void *key_scale, const void *key_min, int64_t ks_sh, int64_t ks_sd, int64_t ks_sg,
-                               const void *value_code, int64_t vc_sh, int64_t vc_st, int64_t vc_sw,
-                               const void *value_scale, const void *value_min, int64_t vs_sh, int64_t vs_st, int64_t vs_sg,
-                               int stats_dtype, int64_t heads, int64_t head_dim,
-                               int k_bits, int v_bits, int group_size, int64_t start, int64_t stop,
-                               void *out_key, void *out_value, int out_dtype,
-                               int64_t o_st, int64_t o_sh, int64_t o_sd, int64_t output_offset,
-                               uc_stream_t stream) {
+namespace uc {
+namespace {
+
+int dequant(const void *key_code, int64_t kc_sh, int64_t kc_sd, int64_t kc_sw,
+            const void *key_scale, const void *key_min, int64_t ks_sh, int64_t ks_sd, int64_t ks_sg,
+            const void *value_code, int64_t vc_sh, int64_t vc_st, int64_t vc_sw,
+            const void *value_scale, const void *value_min, int64_t vs_sh, int64_t vs_st, int64_t vs_sg,
+            int stats_dtype, int64_t heads, int64_t head_dim,
+            int k_bits, int v_bits, int group_size, int64_t start, int64_t stop,
+            void *out_key, void *out_value, int out_dtype,
+            int64_t o_st, int64_t o_sh, int64_t o_sd, int64_t output_offset,
+            const void *res_key, const void *res_value, int64_t res_rows, const char *entry,
+            uc_stream_t stream) {
   UC_REQUIRE(valid_dtype(stats_dtype) && valid_dtype(out_dtype), "uc_kivi_dequant: unknown dtype code");
   UC_REQUIRE(k_bits == 2 || k_bits == 4 || k_bits == 8, "KIVI physical cache supports 2, 4, or 8 bit payloads");
   UC_REQUIRE(v_bits == 2 || v_bits == 4 || v_bits == 8, "KIVI physical cache supports 2, 4, or 8 bit payloads");
@@ -1317,7 +1349,7 @@ extern "C" int uc_kivi_dequant(const void *key_code, int64_t kc_sh, int64_t kc_s
   UC_REQUIRE(key_code == nullptr || out_key != nullptr, "uc_kivi_dequant: missing key output");
   UC_REQUIRE(value_code == nullptr || out_value != nullptr, "uc_kivi_dequant: missing value output");
   const int64_t count = stop - start;
-  if (count == 0) return UC_OK;
+  if (count == 0 && res_rows == 0) return UC_OK;
   DequantArgs a{};
   a.key_code = key_code; a.kc_sh = kc_sh; a.kc_sd = kc_sd; a.kc_sw = kc_sw;
   a.key_scale = key_scale; a.key_min = key_min; a.ks_sh = ks_sh; a.ks_sd = ks_sd; a.ks_sg = ks_sg;
@@ -1331,7 +1363,22 @@ extern "C" int uc_kivi_dequant(const void *key_code, int64_t kc_sh, int64_t kc_s
   a.lg = group_size == 16 ? 4 : group_size == 32 ? 5 : group_size == 64 ? 6 : 7;
   a.group = group_size;
   a.sd = stats_dtype; a.od = out_dtype;
+  a.res_key = res_key; a.res_value = res_value; a.res_rows = res_rows;
   hipStream_t s = as_stream(stream);
+  // the dense rows by themselves, where no launch below takes them along
+  auto residual = [&] {
+    if (res_rows == 0) return;
+    const int64_t per_tensor = res_rows * heads * head_dim;
+    const dim3 grid(static_cast<unsigned>(ceil_div(2 * per_tensor, int64_t(256))));
+    if (out_dtype == UC_FP32)
+      hipLaunchKernelGGL((copy_residual_kernel<uint32_t>), grid, dim3(256), 0, s, a, per_tensor);
+    else
+      hipLaunchKernelGGL((copy_residual_kernel<uint16_t>), grid, dim3(256), 0, s, a, per_tensor);
+  };
+  if (count == 0) {
+    residual();
+    return check_launch(entry);
+  }
   // native 2/4-bit layout with pairwise-aligned unit-stride output rows
   const int out_bytes = out_dtype == UC_FP32 ? 4 : 2;
   const bool out_ok = o_sd == 1 && o_st % 2 == 0 && o_sh % 2 == 0 && head_dim % 32 == 0 &&
@@ -1363,16 +1410,23 @@ extern "C" int uc_kivi_dequant(const void *key_code, int64_t kc_sh, int64_t kc_s
         const int64_t runs = ceil_div(words, int64_t(kDqOctetWords));
         const int64_t key_blocks = ceil_div(heads * runs * (head_dim / 8), int64_t(256));
         const int64_t value_blocks = ceil_div(heads * count * (head_dim * v_bits / 32), int64_t(256));
-        const dim3 grid(static_cast<unsigned>(key_blocks + value_blocks));
+        // the dense rows as well, where they move in 16-byte units: a cache of
+        // 20353 tokens and 32 dense rows was three launches and 18.0 us
+        const bool along = res_rows > 0 && aligned(res_key, 16) && aligned(res_value, 16);
+        const int64_t res_blocks = along ? ceil_div(2 * (res_rows * heads * head_dim / 8), int64_t(256)) : 0;
+        const dim3 grid(static_cast<unsigned>(key_blocks + value_blocks + res_blocks));
         auto go_kv = [&](auto sd_tag) {
           constexpr int SD = decltype(sd_tag)::value;
           if (k_bits == 2)
-            hipLaunchKernelGGL((dequant_kv_kernel<2, OD, SD, true>), grid, dim3(256), 0, s, a, runs, key_blocks);
+            hipLaunchKernelGGL((dequant_kv_kernel<2, OD, SD, true>), grid, dim3(256), 0, s, a, runs, key_blocks,
+                               value_blocks);
           else
-            hipLaunchKernelGGL((dequant_kv_kernel<4, OD, SD, true>), grid, dim3(256), 0, s, a, runs, key_blocks);
+            hipLaunchKernelGGL((dequant_kv_kernel<4, OD, SD, true>), grid, dim3(256), 0, s, a, runs, key_blocks,
+                               value_blocks);
         };
         if (stats_dtype == UC_BF16) go_kv(std::integral_constant<int, UC_BF16>{});
         else go_kv(std::integral_constant<int, UC_FP16>{});
+        if (!along) residual();
         return;
       }
       if (octet) {
@@ -1413,15 +1467,56 @@ extern "C" int uc_kivi_dequant(const void *key_code, int64_t kc_sh, int64_t kc_s
         if (vec) go(std::true_type{});
         else go(std::false_type{});
       }
+      residual();
     });
-    return check_launch("uc_kivi_dequant");
+    return check_launch(entry);
   }
   UC_DISPATCH_BITS(k_bits, KB, [&] {
     UC_DISPATCH_BITS(v_bits, VB, [&] {
       hipLaunchKernelGGL((kivi_dequant_kernel<KB, VB>), dim3(blocks), dim3(256), 0, s, a);
     });
   });
-  return check_launch("uc_kivi_dequant");
+  residual();
+  return check_launch(entry);
+}
+
+}  // namespace
+}  // namespace uc
+
+extern "C" int uc_kivi_dequant(const void *key_code, int64_t kc_sh, int64_t kc_sd, int64_t kc_sw,
+                               const void *key_scale, const void *key_min, int64_t ks_sh, int64_t ks_sd, int64_t ks_sg,
+                               const void *value_code, int64_t vc_sh, int64_t vc_st, int64_t vc_sw,
+                               const void *value_scale, const void *value_min, int64_t vs_sh, int64_t vs_st, int64_t vs_sg,
+                               int stats_dtype, int64_t heads, int64_t head_dim,
+                               int k_bits, int v_bits, int group_size, int64_t start, int64_t stop,
+                               void *out_key, void *out_value, int out_dtype,
+                               int64_t o_st, int64_t o_sh, int64_t o_sd, int64_t output_offset,
+                               uc_stream_t stream) {
+  return dequant(key_code, kc_sh, kc_sd, kc_sw, key_scale, key_min, ks_sh, ks_sd, ks_sg, value_code, vc_sh,
+                 vc_st, vc_sw, value_scale, value_min, vs_sh, vs_st, vs_sg, stats_dtype, heads, head_dim,
+                 k_bits, v_bits, group_size, start, stop, out_key, out_value, out_dtype, o_st, o_sh, o_sd,
+                 output_offset, nullptr, nullptr, 0, "uc_kivi_dequant", stream);
+}
+
+extern "C" int uc_kivi_restore(const void *key_code, int64_t kc_sh, int64_t kc_sd, int64_t kc_sw,
+                               const void *key_scale, const void *key_min, int64_t ks_sh, int64_t ks_sd, int64_t ks_sg,
+                               const void *value_code, int64_t vc_sh, int64_t vc_st, int64_t vc_sw,
+                               const void *value_scale, const void *value_min, int64_t vs_sh, int64_t vs_st, int64_t vs_sg,
+                               int stats_dtype, int64_t heads, int64_t head_dim,
+                               int k_bits, int v_bits, int group_size, int64_t start, int64_t stop,
+                               void *out_key, void *out_value, int out_dtype,
+                               int64_t o_st, int64_t o_sh, int64_t o_sd, int64_t output_offset,
+                               const void *res_key, const void *res_value, int64_t res_rows,
+                               uc_stream_t stream) {
+  UC_REQUIRE(res_rows >= 0 && (res_rows == 0 || (res_key != nullptr && res_value != nullptr)),
+             "uc_kivi_restore: missing dense rows");
+  UC_REQUIRE(out_key != nullptr && out_value != nullptr, "uc_kivi_restore: missing output");
+  UC_REQUIRE(heads > 0 && head_dim > 0 && res_rows * heads * head_dim <= (int64_t(1) << 30),
+             "uc_kivi_restore: too many dense rows for one call (%lld)", (long long)res_rows);
+  return dequant(key_code, kc_sh, kc_sd, kc_sw, key_scale, key_min, ks_sh, ks_sd, ks_sg, value_code, vc_sh,
+                 vc_st, vc_sw, value_scale, value_min, vs_sh, vs_st, vs_sg, stats_dtype, heads, head_dim,
+                 k_bits, v_bits, group_size, start, stop, out_key, out_value, out_dtype, o_st, o_sh, o_sd,
+                 output_offset, res_key, res_value, res_rows, "uc_kivi_restore", stream);
 }
 
 extern "C" int uc_kivi_fake_quant(const void *data, int64_t st, int64_t sh, int64_t sd,

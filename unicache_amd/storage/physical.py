@@ -672,12 +672,16 @@ class PackedKIVICache:
             return
         ref = out_key if out_key is not None else out_value
         device = nat.require_device(self.key_code, ref, what="KIVI dequantization")
-        kcs, kss, vcs, vss = self._code_strides()
         if out_key is not None and out_value is not None:
             if out_key.stride() != out_value.stride() or out_key.dtype != out_value.dtype:
                 raise ValueError("KIVI dequantization output workspace has an invalid layout")
+        self._restore("uc_kivi_dequant", device, out_key, out_value, start, stop, output_offset)
+
+    def _restore(self, entry, device, out_key, out_value, start, stop, output_offset, *residual) -> None:
+        ref = out_key if out_key is not None else out_value
+        kcs, kss, vcs, vss = self._code_strides()
         nat.call(
-            "uc_kivi_dequant",
+            entry,
             nat.ptr(self.key_code) if out_key is not None else None, *map(int, kcs),
             self.key_scale.data_ptr(), self.key_minimum.data_ptr(), *map(int, kss),
             nat.ptr(self.value_code) if out_value is not None else None, *map(int, vcs),
@@ -685,7 +689,7 @@ class PackedKIVICache:
             nat.dtype_code(self.key_scale.dtype), self.num_kv_heads, self.head_dim,
             self.k_bits, self.v_bits, self.group_size, int(start), int(stop),
             nat.ptr(out_key), nat.ptr(out_value), nat.dtype_code(ref.dtype),
-            *map(int, ref.stride()), int(output_offset), nat.stream(device),
+            *map(int, ref.stride()), int(output_offset), *residual, nat.stream(device),
         )
 
     def dequantize(self, dtype: torch.dtype | None = None) -> tuple[torch.Tensor, torch.Tensor]:
@@ -698,6 +702,16 @@ class PackedKIVICache:
         shape = (total, self.num_kv_heads, self.head_dim)
         key = torch.empty(shape, dtype=dtype, device=self.key_code.device)
         value = torch.empty_like(key)
+        dense = self.residual_key, self.residual_value
+        if self.residual_tokens and all(
+            x.device == key.device and x.dtype == dtype and x.is_contiguous() and not x.requires_grad
+            and x.shape == (self.residual_tokens, *shape[1:]) and x.numel() <= 1 << 30
+            for x in dense
+        ):  # compact rows of the wanted type: the same launch copies them
+            device = nat.require_device(self.key_code, key, what="KIVI dequantization")
+            self._restore("uc_kivi_restore", device, key, value, 0, self.quantized_tokens, 0,
+                          dense[0].data_ptr(), dense[1].data_ptr(), self.residual_tokens)
+            return key, value
         self.dequantize_into(key, value, start=0, stop=self.quantized_tokens, output_offset=0)
         key[self.quantized_tokens:].copy_(self.residual_key)
         value[self.quantized_tokens:].copy_(self.residual_value)

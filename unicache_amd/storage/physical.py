@@ -254,29 +254,30 @@ def _native_block(capacity: int, heads: int, head_dim: int, k_bits: int, v_bits:
     view op each), the storage addresses, and the ids tensor (or None).  The
     few host operations matter: from_dense runs once per materialised segment."""
 
-    specs = _native_specs(capacity, heads, head_dim, k_bits, v_bits, group_size)
-    if ids_dtype is not None:
-        specs.append(((ids_len,), ids_dtype))
-    offsets, total = [], 0
-    for shape, dtype in specs:
-        offsets.append(total)
-        total += -(-math.prod(shape) * dtype.itemsize // _CARVE_ALIGN) * _CARVE_ALIGN
-    buf = torch.empty(max(total, _CARVE_ALIGN), dtype=torch.uint8, device=device)
-    i32, f16 = buf.view(torch.int32), buf.view(torch.float16)
     d, nw, ng = head_dim, capacity * k_bits // 32, capacity // group_size
     vw, vg = head_dim * v_bits // 32, head_dim // group_size
-    o = offsets
+    # bytes of the tensors of _native_specs, in order
+    ks, vs = 2 * heads * ng * d, 2 * heads * capacity * vg
+    sizes = [4 * heads * nw * d, ks, ks, 4 * heads * capacity * vw, vs, vs]
+    if ids_dtype is not None:
+        sizes.append(ids_len * ids_dtype.itemsize)
+    o, total = [], 0
+    for size in sizes:
+        o.append(total)
+        total += -(-size // _CARVE_ALIGN) * _CARVE_ALIGN
+    i32 = torch.empty(max(total, _CARVE_ALIGN) // 4, dtype=torch.int32, device=device)
+    f16 = i32.view(torch.float16)
     views = (i32.as_strided((heads, d, nw), (nw * d, 1, d), o[0] // 4),
              f16.as_strided((heads, d, ng), (ng * d, 1, d), o[1] // 2),
              f16.as_strided((heads, d, ng), (ng * d, 1, d), o[2] // 2),
              i32.as_strided((heads, capacity, vw), (capacity * vw, vw, 1), o[3] // 4),
              f16.as_strided((heads, capacity, vg), (capacity * vg, vg, 1), o[4] // 2),
              f16.as_strided((heads, capacity, vg), (capacity * vg, vg, 1), o[5] // 2))
-    base = buf.data_ptr()
+    base = i32.data_ptr()
     ids = None
     if ids_dtype is not None:
-        ids = buf.view(ids_dtype).as_strided((ids_len,), (1,), o[6] // ids_dtype.itemsize)
-    return views, tuple(base + off for off in o[:6]), ids
+        ids = i32.view(ids_dtype).as_strided((ids_len,), (1,), o[6] // ids_dtype.itemsize)
+    return views, tuple([base + off for off in o[:6]]), ids
 
 
 def _pack_native(key: torch.Tensor, value: torch.Tensor, *, k_bits: int, v_bits: int, group_size: int,
@@ -405,13 +406,12 @@ class PackedKIVICache:
         requested_residual = min(tokens, max(0, int(residual_length)))
         # keep any incomplete prefix group in the residual (physical.py:258-263)
         quantized = ((tokens - requested_residual) // group_size) * group_size
-        q_key, q_value = key[:quantized], value[:quantized]
         kernel_native_layout = bool(backend == "cuda" and quantized and k_bits in {2, 4} and v_bits in {2, 4})
         if kernel_native_layout:
             return cls._from_dense_native(key, value, quantized, logical_token_ids, token_type_id, k_bits, v_bits,
                                           group_size)
         if quantized:
-            packed = _pack_reference_layout(q_key, q_value, k_bits=k_bits, v_bits=v_bits, group_size=group_size)
+            packed = _pack_reference_layout(key[:quantized], value[:quantized], k_bits=k_bits, v_bits=v_bits, group_size=group_size)
             key_code, key_scale, key_minimum, value_code, value_scale, value_minimum = packed
         else:
             nat.require_device(key, value, what="KIVI physical cache")
@@ -462,20 +462,25 @@ class PackedKIVICache:
         # the residual rows as compact copies, so a suffix view does not pin
         # the whole dense segment (physical.py:316-319), and the ids: one
         # launch for the three copies
-        tail_k, tail_v = key[quantized:], value[quantized:]
-        res_k = torch.empty(tail_k.shape, dtype=key.dtype, device=device)
-        res_v = torch.empty(tail_v.shape, dtype=value.dtype, device=device)
+        shape = (int(key.shape[0]) - quantized, heads, head_dim)
+        res_k = torch.empty(shape, dtype=key.dtype, device=device)
+        res_v = torch.empty(shape, dtype=value.dtype, device=device)
+        row = heads * head_dim * key.element_size()
+        tail_k, tail_v, skip = key, value, quantized * row  # of contiguous tensors by address: no views
+        if not (key.is_contiguous() and value.is_contiguous()):
+            tail_k, tail_v, skip = key[quantized:], value[quantized:], 0
         if tail_k.is_contiguous() and tail_v.is_contiguous() and (not ids_here or ids.is_contiguous()):
-            nbytes = tail_k.numel() * tail_k.element_size()
-            spans = [tail_k.data_ptr(), res_k.data_ptr(), nbytes, tail_v.data_ptr(), res_v.data_ptr(), nbytes]
+            nbytes = shape[0] * row
+            spans = [tail_k.data_ptr() + skip, res_k.data_ptr(), nbytes,
+                     tail_v.data_ptr() + skip, res_v.data_ptr(), nbytes]
             if ids_here:
                 spans += [ids.data_ptr(), ids_slot.data_ptr(), ids.numel() * ids.element_size()]
             table = (ctypes.c_int64 * len(spans))(*spans)
             nat.call("uc_copy_spans", ctypes.addressof(table), len(spans) // 3, stream)
             ids_copy = ids_slot if ids_here else ids.clone()
         else:
-            res_k.copy_(tail_k)
-            res_v.copy_(tail_v)
+            res_k.copy_(key[quantized:])
+            res_v.copy_(value[quantized:])
             ids_copy = ids_slot.copy_(ids) if ids_here else ids.clone()
         return cls(*views, res_k, res_v, ids_copy, int(token_type_id), int(k_bits), int(v_bits), int(group_size),
                    quantized, head_dim, heads, "cuda", True)

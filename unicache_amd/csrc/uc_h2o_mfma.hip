@@ -434,7 +434,8 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3)))
   }
   // every row of the wave exists and rows take whole stores: full tiles end with
   // exactly 16 stores, which acquire_past_stores counts on
-  const bool whole = vec && row0 + kHsRowsPerWave <= p.rows;
+  // (a scalar: the branches on it hold the barrier)
+  const bool whole = __builtin_amdgcn_readfirstlane(vec && row0 + kHsRowsPerWave <= p.rows) != 0;
   // where this lane's first store of a block pair goes: row n & 7 of 16 qb,
   // keys 4k .. + 3 of the pair's first (n < 8) or second block; its other store
   // is 8 rows on (rows are contiguous: [Hq][Lq] of one KV head)

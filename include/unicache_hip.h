@@ -251,8 +251,7 @@ int uc_kivi_attn_decode(const uc_kivi_item *item_host, int bits, int group_size,
  * GPU's scratch: calls that overlap on one GPU (different streams or host
  * threads without ordering) race and give wrong results.  The device current
  * on the calling thread must be the one that owns the item's tensors and
- * `stream`.  Results equal bit for bit those of uc_kivi_attn_decode with a
- * workspace of uc_kivi_decode_workspace_bytes(1, ...) bytes.
+ * `stream`.  Results equal uc_kivi_attn_decode's bit for bit.
  */
 int uc_kivi_attn_decode_static(const uc_kivi_item *item_host, int bits, int group_size,
                                int64_t heads_q, int64_t heads_kv, int64_t head_dim, int64_t query_len,
@@ -310,6 +309,31 @@ int uc_kivi_attn_decode_segments(const uc_kivi_item *items_device, int64_t n_ite
                                  int q_dtype, int res_dtype, int out_dtype, float sm_scale,
                                  int64_t max_quantized_tokens, int64_t max_residual_tokens,
                                  void *workspace, int64_t workspace_bytes, uc_stream_t stream);
+
+/*
+ * The decode calls above, free to split finer: a launch too small to fill the
+ * GPU takes smaller splits, into more partials, and ends sooner (one 2048-token
+ * segment 16.7 instead of 20.5 us, call to call).  The split size follows from
+ * the launch as a whole (n_items, heads_kv, bits and the largest token counts),
+ * so the last bits of a segment's result may differ from those of the calls
+ * above and from those of the same segment in a launch of another size.  They
+ * never depend on the workspace, which must hold
+ * uc_kivi_decode_preferred_workspace_bytes(n_items, ...) bytes.
+ * Exactly one of items_host and items_device is given:
+ *   items_host:   the 1..8 segments of one query as in
+ *                 uc_kivi_attn_decode_segments_host (segments_per_query ==
+ *                 n_items; the largest token counts are taken from the items);
+ *                 one item without residual strides as in uc_kivi_attn_decode.
+ *   items_device: as in uc_kivi_attn_decode_segments, or with
+ *                 segments_per_query 1 as in uc_kivi_attn_decode_batch.
+ * No reference counterpart.
+ */
+int uc_kivi_attn_decode_fine(const uc_kivi_item *items_host, const uc_kivi_item *items_device, int64_t n_items,
+                             int64_t segments_per_query, int bits, int group_size,
+                             int64_t heads_q, int64_t heads_kv, int64_t head_dim, int64_t query_len,
+                             int q_dtype, int res_dtype, int out_dtype, float sm_scale,
+                             int64_t max_quantized_tokens, int64_t max_residual_tokens,
+                             void *workspace, int64_t workspace_bytes, uc_stream_t stream);
 
 /*
  * Attention for long queries (image editing: group*query_len rows per KV head
@@ -684,11 +708,8 @@ int64_t uc_kivi_decode_workspace_bytes(int64_t n_items, int bits, int group_size
                                        int64_t max_quantized_tokens, int64_t max_residual_tokens);
 
 /*
- * Bytes of workspace with which the same calls are fastest: launches too small
- * to fill the GPU then split their segments finer, into more partials.  At
- * least uc_kivi_decode_workspace_bytes and at most about 3.3 MB more.  A call
- * with less workspace than this is valid and splits coarser; its results
- * differ in the rounding of the partials only.
+ * The same for uc_kivi_attn_decode_fine: at least
+ * uc_kivi_decode_workspace_bytes and at most about 3.3 MB more.
  */
 int64_t uc_kivi_decode_preferred_workspace_bytes(int64_t n_items, int bits, int group_size, int64_t heads_q,
                                                  int64_t heads_kv, int64_t head_dim, int64_t query_len,

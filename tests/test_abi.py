@@ -101,6 +101,26 @@ def test_preferred_decode_workspace():
         nat.decode_preferred_workspace_bytes(-1, 2, 32, 28, 4, 128, 1, 64, 0)
 
 
+def test_fine_decode_validation():
+    item = nat.KiviItem()
+    item.quantized_tokens = 64
+    args = (2, 32, 28, 4, 128, 1, nat.UC_BF16, nat.UC_BF16, nat.UC_BF16, 0.1)
+    with pytest.raises(ValueError, match="host or in device"):
+        nat.call("uc_kivi_attn_decode_fine", None, None, 1, 1, *args, 64, 0, None, 0, None)
+    with pytest.raises(ValueError, match="host or in device"):
+        nat.call("uc_kivi_attn_decode_fine", item, 16, 1, 1, *args, 64, 0, None, 0, None)
+    with pytest.raises(ValueError, match="segments of one query"):
+        nat.call("uc_kivi_attn_decode_fine", item, None, 1, 2, *args, 64, 0, None, 0, None)
+    with pytest.raises(ValueError, match="groups of 2"):
+        nat.call("uc_kivi_attn_decode_fine", None, 16, 3, 2, *args, 64, 0, None, 0, None)
+    with pytest.raises(ValueError, match="workspace too small"):
+        nat.call("uc_kivi_attn_decode_fine", None, 16, 3, 1, *args, 64, 0, None, 0, None)
+    with pytest.raises(ValueError, match="16-byte aligned"):  # strided rows as in uc_kivi_attn_decode_segments_host
+        item.quantized_tokens, item.residual_tokens, item.residual_key, item.residual_value = 0, 4, 8, 8
+        item.residual_token_stride, item.residual_head_stride = 512, 128
+        nat.call("uc_kivi_attn_decode_fine", item, None, 1, 1, *args, 0, 0, None, 0, None)
+
+
 def test_editing_validation():
     item = nat.KiviItem()
     item.quantized_tokens = 64

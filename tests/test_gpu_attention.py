@@ -192,32 +192,56 @@ def test_decode_query_rows_around_the_fold(device, hq, hkv, lq):
         check_summary(out, lse, seg, q, what=f"Hq {hq} Hkv {hkv} Lq {lq} T {tokens}")
 
 
-@pytest.mark.parametrize("bits,group,tokens,heads", [(2, 32, 255 + 32, 4), (2, 64, 256 + 64, 4), (2, 32, 2100, 2),
-                                                     (4, 64, 1999, 4), (2, 32, 33000, 1), (4, 128, 9000, 8)])
-def test_decode_split_sizes_by_workspace(device, bits, group, tokens, heads):
-    # a small launch splits its segments finer when the workspace allows it
-    # (uc_kivi_decode_preferred_workspace_bytes) and keeps 8 super-tiles per
-    # split with the least workspace: both against the oracle, from one
-    # super-tile (and one token more) to 129 of them on one KV head
-    import ctypes
-
+# packed tokens with group 32 and residual 100: none of two super-tiles (160), one (256 at 2 bits) and one group
+# more (288), eight; 16 of 128 tokens at 4 bits; 129 super-tiles on one KV head
+@pytest.mark.parametrize("bits,group,tokens,heads,packed", [(2, 32, 287, 4, 160), (2, 32, 356, 4, 256),
+                                                            (2, 32, 388, 4, 288), (2, 32, 2148, 2, 2048),
+                                                            (4, 64, 1999, 4, 1856), (2, 32, 33000, 1, 32896),
+                                                            (4, 128, 9000, 8, 8832)])
+def test_decode_results_do_not_depend_on_workspace(device, bits, group, tokens, heads, packed):
+    # the calls that do not ask for finer splits give the same bits whatever the
+    # workspace, and the call without one gives them too; the finer splits of a
+    # small launch against the oracle, the same bits again with a larger workspace
     cache, seg = _pair(tokens, 150, bits, group, 100, device, heads=heads)
+    assert cache.quantized_tokens == packed
     q = queries(1, heads=7 * heads, seed=151)
     qd = q.to(device)
     args = (bits, group, 7 * heads, heads, 128, 1)
     tr = cache.residual_tokens
-    sizes = [f(1, *args, cache.quantized_tokens, tr)
-             for f in (nat.decode_workspace_bytes, nat.decode_preferred_workspace_bytes)]
-    assert sizes[1] >= sizes[0]
-    for nbytes in sizes:
+    least, preferred = [f(1, *args, packed, tr)
+                        for f in (nat.decode_workspace_bytes, nat.decode_preferred_workspace_bytes)]
+    super_tiles = -(-packed // (16 * (32 // bits)))
+    assert preferred > least if super_tiles > 1 else preferred == least
+
+    def summary(entry, nbytes):
         out, lse = torch.empty_like(qd), torch.empty((7 * heads, 1), dtype=torch.float32, device=device)
         item = cache.native_item(qd.data_ptr(), out.data_ptr(), lse.data_ptr(),
                                  residual_key_ptr=cache.residual_key.data_ptr(),
                                  residual_value_ptr=cache.residual_value.data_ptr(), residual_tokens=tr)
+        types = (nat.UC_BF16, nat.UC_BF16, nat.UC_BF16, 1.0 / math.sqrt(128))
         ws = nat.workspace(device, nbytes)
-        nat.call("uc_kivi_attn_decode", ctypes.byref(item), *args, nat.UC_BF16, nat.UC_BF16, nat.UC_BF16,
-                 1.0 / math.sqrt(128), ws.data_ptr(), nbytes, nat.stream(device))
-        check_summary(out, lse, seg, q, what=f"{nbytes} bytes of workspace")
+        room = (ws.data_ptr(), nbytes, nat.stream(device))
+        if entry == "uc_kivi_attn_decode_static":
+            nat.call(entry, item, *args, *types, nat.stream(device))
+        elif entry == "uc_kivi_attn_decode_segments_host":
+            nat.call(entry, item, 1, *args, *types, *room)
+        elif entry == "uc_kivi_attn_decode":
+            nat.call(entry, item, *args, *types, *room)
+        else:
+            nat.call(entry, item, None, 1, 1, *args, *types, 0, 0, *room)
+        check_summary(out, lse, seg, q, what=f"{entry} with {nbytes} bytes of workspace")
+        return out, lse
+
+    want = summary("uc_kivi_attn_decode", least)
+    for entry, nbytes in (("uc_kivi_attn_decode", preferred), ("uc_kivi_attn_decode", 8 << 20),
+                          ("uc_kivi_attn_decode_static", 0), ("uc_kivi_attn_decode_segments_host", 8 << 20)):
+        got = summary(entry, nbytes)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), (entry, nbytes)
+    fine = summary("uc_kivi_attn_decode_fine", preferred)
+    more = summary("uc_kivi_attn_decode_fine", 8 << 20)
+    assert torch.equal(fine[0], more[0]) and torch.equal(fine[1], more[1])
+    with pytest.raises(ValueError, match="workspace too small"):
+        summary("uc_kivi_attn_decode_fine", 4)
 
 
 def test_decode_is_deterministic(device):

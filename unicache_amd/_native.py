@@ -137,6 +137,10 @@ _SIGNATURES = {
         _I,
         [ctypes.POINTER(KiviItem), _I, _I, _L, _L, _L, _L, _I, _I, _I, _F, _P, _L, _P],
     ),
+    "uc_kivi_attn_decode_fine": (
+        _I,
+        [ctypes.POINTER(KiviItem), _P, _L, _L, _I, _I, _L, _L, _L, _L, _I, _I, _I, _F, _L, _L, _P, _L, _P],
+    ),
     "uc_kivi_attn_decode_static": (
         _I,
         [ctypes.POINTER(KiviItem), _I, _I, _L, _L, _L, _L, _I, _I, _I, _F, _P],
@@ -327,7 +331,7 @@ def decode_workspace_bytes(n_items, bits, group_size, heads_q, heads_kv, head_di
 @functools.lru_cache(maxsize=256)
 def decode_preferred_workspace_bytes(n_items, bits, group_size, heads_q, heads_kv, head_dim, query_len, max_tq,
                                      max_tr) -> int:
-    """The decode workspace with which small launches are free to split finer."""
+    """The workspace of uc_kivi_attn_decode_fine."""
 
     size = int(lib().uc_kivi_decode_preferred_workspace_bytes(n_items, bits, group_size, heads_q, heads_kv, head_dim,
                                                               query_len, max_tq, max_tr))

@@ -401,7 +401,7 @@ int decode_common(const uc_kivi_item *items_dev, const uc_kivi_item *single, int
                   int group_size, int64_t Hq, int64_t Hkv, int64_t D, int64_t Lq, int q_dtype,
                   int res_dtype, int out_dtype, float sm_scale, int64_t max_tq, int64_t max_tr,
                   void *workspace, int64_t workspace_bytes, hipStream_t stream, const char *name,
-                  int64_t segs = 1) {
+                  int64_t segs = 1, bool fine = false) {
   UC_REQUIRE(bits == 2 || bits == 4, "%s: packed decode supports 2 or 4 bit codes", name);
   UC_REQUIRE(group_size == 16 || group_size == 32 || group_size == 64 || group_size == 128,
              "%s: group_size must be 16, 32, 64 or 128", name);
@@ -425,7 +425,7 @@ int decode_common(const uc_kivi_item *items_dev, const uc_kivi_item *single, int
     UC_REQUIRE(single == nullptr || (reinterpret_cast<uintptr_t>(single->query) & 15) == 0,
                "%s: query must be 16-byte aligned", name);
     return launch_decode_mfma(items_dev, single, n_items, bits, group_size, Hq, Hkv, Lq, q_dtype, res_dtype,
-                              out_dtype, sm_scale, max_tq, max_tr, kDecodeMfmaNst, segs, workspace,
+                              out_dtype, sm_scale, max_tq, max_tr, kDecodeMfmaNst, segs, fine, workspace,
                               workspace_bytes, stream);
   }
   const int64_t sp_packed = ceil_div(max_tq, kDecodeSplitTokens);
@@ -471,6 +471,51 @@ int decode_common(const uc_kivi_item *items_dev, const uc_kivi_item *single, int
   else
     hipLaunchKernelGGL((decode_combine_kernel<false>), cgrid, dim3(128), 0, stream, items_dev, one, c);
   return check_launch(name);
+}
+
+// One query group over n_items segments given in host memory.
+int decode_segments_host(const uc_kivi_item *items_host, int64_t n_items, int bits, int group_size, int64_t heads_q,
+                         int64_t heads_kv, int64_t head_dim, int64_t query_len, int q_dtype, int res_dtype,
+                         int out_dtype, float sm_scale, void *workspace, int64_t workspace_bytes, hipStream_t stream,
+                         bool fine) {
+  clear_error();
+  constexpr int64_t kMaxHostItems = 8;
+  UC_REQUIRE(items_host != nullptr && n_items >= 1 && n_items <= kMaxHostItems,
+             "uc_kivi_attn_decode_segments_host: 1..%lld items", (long long)kMaxHostItems);
+  UC_REQUIRE(heads_kv > 0 && head_dim > 0, "uc_kivi_attn_decode_segments_host: bad head shape");
+  uc_kivi_item items[kMaxHostItems];
+  int64_t max_tq = 0, max_tr = 0;
+  for (int64_t i = 0; i < n_items; ++i) {
+    uc_kivi_item it = items_host[i];
+    // one query group: every segment reads the first item's query; its out / lse get the result
+    it.query = items_host[0].query;
+    it.out = items_host[0].out;
+    it.lse = items_host[0].lse;
+    UC_REQUIRE(it.quantized_tokens >= 0 && it.residual_tokens >= 0 && it.quantized_tokens % group_size == 0,
+               "uc_kivi_attn_decode_segments_host: item %lld: bad token counts", (long long)i);
+    UC_REQUIRE(it.quantized_tokens == 0 ||
+                   (it.key_code && it.key_scale && it.key_min && it.value_code && it.value_scale && it.value_min &&
+                    (it.packed_capacity == 0 ||
+                     (it.packed_capacity >= it.quantized_tokens && it.packed_capacity % group_size == 0))),
+               "uc_kivi_attn_decode_segments_host: item %lld: packed tensors or capacity", (long long)i);
+    if (it.residual_tokens) {
+      int64_t ts, hs;
+      residual_strides(it, heads_kv, head_dim, ts, hs);
+      UC_REQUIRE(it.residual_key && it.residual_value &&
+                     ((reinterpret_cast<uintptr_t>(it.residual_key) | reinterpret_cast<uintptr_t>(it.residual_value)) &
+                      15) == 0 && ts > 0 && hs >= 0 && ts % 8 == 0 && hs % 8 == 0,
+                 "uc_kivi_attn_decode_segments_host: item %lld: residual rows must be 16-byte aligned with strides "
+                 "in multiples of 8 elements", (long long)i);
+      UC_REQUIRE(((it.residual_tokens - 1) * ts + (heads_kv - 1) * hs + head_dim) * 2 < (int64_t(1) << 31),
+                 "uc_kivi_attn_decode_segments_host: item %lld: residual rows span 2 GiB or more", (long long)i);
+    }
+    max_tq = max(max_tq, it.quantized_tokens);
+    max_tr = max(max_tr, it.residual_tokens);
+    items[i] = it;
+  }
+  return decode_common(nullptr, items, n_items, bits, group_size, heads_q, heads_kv, head_dim, query_len, q_dtype,
+                       res_dtype, out_dtype, sm_scale, max_tq, max_tr, workspace, workspace_bytes, stream,
+                       "uc_kivi_attn_decode_segments_host", n_items, fine);
 }
 
 }  // namespace
@@ -526,44 +571,38 @@ extern "C" int uc_kivi_attn_decode_segments_host(const uc_kivi_item *items_host,
                                                  int64_t head_dim, int64_t query_len, int q_dtype, int res_dtype,
                                                  int out_dtype, float sm_scale, void *workspace,
                                                  int64_t workspace_bytes, uc_stream_t stream) {
-  clear_error();
-  constexpr int64_t kMaxHostItems = 8;
-  UC_REQUIRE(items_host != nullptr && n_items >= 1 && n_items <= kMaxHostItems,
-             "uc_kivi_attn_decode_segments_host: 1..%lld items", (long long)kMaxHostItems);
-  UC_REQUIRE(heads_kv > 0 && head_dim > 0, "uc_kivi_attn_decode_segments_host: bad head shape");
-  uc_kivi_item items[kMaxHostItems];
-  int64_t max_tq = 0, max_tr = 0;
-  for (int64_t i = 0; i < n_items; ++i) {
-    uc_kivi_item it = items_host[i];
-    // one query group: every segment reads the first item's query; its out / lse get the result
-    it.query = items_host[0].query;
-    it.out = items_host[0].out;
-    it.lse = items_host[0].lse;
-    UC_REQUIRE(it.quantized_tokens >= 0 && it.residual_tokens >= 0 && it.quantized_tokens % group_size == 0,
-               "uc_kivi_attn_decode_segments_host: item %lld: bad token counts", (long long)i);
-    UC_REQUIRE(it.quantized_tokens == 0 ||
-                   (it.key_code && it.key_scale && it.key_min && it.value_code && it.value_scale && it.value_min &&
-                    (it.packed_capacity == 0 ||
-                     (it.packed_capacity >= it.quantized_tokens && it.packed_capacity % group_size == 0))),
-               "uc_kivi_attn_decode_segments_host: item %lld: packed tensors or capacity", (long long)i);
-    if (it.residual_tokens) {
-      int64_t ts, hs;
-      residual_strides(it, heads_kv, head_dim, ts, hs);
-      UC_REQUIRE(it.residual_key && it.residual_value &&
-                     ((reinterpret_cast<uintptr_t>(it.residual_key) | reinterpret_cast<uintptr_t>(it.residual_value)) &
-                      15) == 0 && ts > 0 && hs >= 0 && ts % 8 == 0 && hs % 8 == 0,
-                 "uc_kivi_attn_decode_segments_host: item %lld: residual rows must be 16-byte aligned with strides "
-                 "in multiples of 8 elements", (long long)i);
-      UC_REQUIRE(((it.residual_tokens - 1) * ts + (heads_kv - 1) * hs + head_dim) * 2 < (int64_t(1) << 31),
-                 "uc_kivi_attn_decode_segments_host: item %lld: residual rows span 2 GiB or more", (long long)i);
-    }
-    max_tq = max(max_tq, it.quantized_tokens);
-    max_tr = max(max_tr, it.residual_tokens);
-    items[i] = it;
+  return decode_segments_host(items_host, n_items, bits, group_size, heads_q, heads_kv, head_dim, query_len, q_dtype,
+                              res_dtype, out_dtype, sm_scale, workspace, workspace_bytes, as_stream(stream), false);
+}
+
+extern "C" int uc_kivi_attn_decode_fine(const uc_kivi_item *items_host, const uc_kivi_item *items_device,
+                                        int64_t n_items, int64_t segments_per_query, int bits, int group_size,
+                                        int64_t heads_q, int64_t heads_kv, int64_t head_dim, int64_t query_len,
+                                        int q_dtype, int res_dtype, int out_dtype, float sm_scale,
+                                        int64_t max_quantized_tokens, int64_t max_residual_tokens, void *workspace,
+                                        int64_t workspace_bytes, uc_stream_t stream) {
+  const char *name = "uc_kivi_attn_decode_fine";
+  UC_REQUIRE((items_host == nullptr) != (items_device == nullptr) || n_items == 0,
+             "%s: items in host or in device memory", name);
+  if (items_host != nullptr) {
+    UC_REQUIRE(segments_per_query == n_items, "%s: items in host memory are the segments of one query", name);
+    const uc_kivi_item &it = *items_host;
+    if (n_items != 1 || it.residual_token_stride != 0 || it.residual_head_stride != 0)
+      return decode_segments_host(items_host, n_items, bits, group_size, heads_q, heads_kv, head_dim, query_len,
+                                  q_dtype, res_dtype, out_dtype, sm_scale, workspace, workspace_bytes,
+                                  as_stream(stream), true);
+    UC_REQUIRE(it.quantized_tokens >= 0 && it.residual_tokens >= 0, "%s: negative token count", name);
+    return decode_common(nullptr, items_host, 1, bits, group_size, heads_q, heads_kv, head_dim, query_len, q_dtype,
+                         res_dtype, out_dtype, sm_scale, it.quantized_tokens, it.residual_tokens, workspace,
+                         workspace_bytes, as_stream(stream), name, 1, true);
   }
-  return decode_common(nullptr, items, n_items, bits, group_size, heads_q, heads_kv, head_dim, query_len, q_dtype,
-                       res_dtype, out_dtype, sm_scale, max_tq, max_tr, workspace, workspace_bytes, as_stream(stream),
-                       "uc_kivi_attn_decode_segments_host", n_items);
+  UC_REQUIRE(n_items >= 0, "%s: bad item table", name);
+  UC_REQUIRE(segments_per_query >= 1 && n_items % segments_per_query == 0,
+             "%s: %lld items do not form groups of %lld", name, (long long)n_items, (long long)segments_per_query);
+  UC_REQUIRE(max_quantized_tokens >= 0 && max_residual_tokens >= 0, "%s: negative tokens", name);
+  return decode_common(items_device, nullptr, n_items, bits, group_size, heads_q, heads_kv, head_dim, query_len,
+                       q_dtype, res_dtype, out_dtype, sm_scale, max_quantized_tokens, max_residual_tokens, workspace,
+                       workspace_bytes, as_stream(stream), name, segments_per_query, true);
 }
 
 extern "C" int uc_kivi_qk(const void *query, int q_dtype, int64_t query_len, int64_t heads_q,
@@ -746,5 +785,5 @@ extern "C" int uc_kivi_attn_decode_static(const uc_kivi_item *item_host, int bit
   if (rc != UC_OK) return rc;
   return decode_common(nullptr, item_host, 1, bits, group_size, heads_q, heads_kv, head_dim, query_len, q_dtype,
                        res_dtype, out_dtype, sm_scale, item_host->quantized_tokens, item_host->residual_tokens, ws,
-                       need, as_stream(stream), "uc_kivi_attn_decode_static");
+                       kDecodeScratchBytes, as_stream(stream), "uc_kivi_attn_decode_static");
 }

@@ -1155,9 +1155,9 @@ static void launch_group(bool table, int rd, dim3 grid, hipStream_t stream, cons
 
 // Super-tiles per packed split of a launch.  `nst` per split is the right size
 // for launches of several rounds of workgroup slots (kWgPerCu per CU): there a
-// split's fixed cost counts.  A launch that does not fill one round is bound by
-// the longest split's serial chain instead, so it takes the split size with the
-// least estimated time: the chain's super-tiles at the measured 1.36, 1.8 or
+// split's fixed cost counts.  A `fine` launch that does not fill one round is
+// bound by the longest split's serial chain instead, so it takes the split size
+// with the least estimated time: the chain's super-tiles at the measured 1.36, 1.8 or
 // 2.7 us each with 1, 2 or 3 workgroups on a CU (alone, a wave leaves half its
 // SIMD's issue slots idle; three waves fill them), plus 0.09 us per split that
 // the combine reads, in units of 0.09 us.  Measured, call to call: 8 sequences
@@ -1165,9 +1165,10 @@ static void launch_group(bool table, int rd, dim3 grid, hipStream_t stream, cons
 // 18.1 us (3), one 32768-token segment 21.9 -> 16.2 us (3; 18.6 with 2, 17.2
 // with 4), 8 x 8192 at 4 bits 21.8 -> 18.2 us (3); the estimate picked the
 // fastest or within 0.2 us of it on 15 shapes of 8 to 1024 super-tiles a unit.
-// `workspace_bytes` caps the choice: callers may bring the least workspace.
+// The choice never looks at the size of the workspace, so results do not depend
+// on it.
 static int64_t choose_super_tiles(int64_t nst, int64_t n_items, int64_t Hkv, int bits, int64_t max_tq, int64_t max_tr,
-                                  int64_t segs, int64_t workspace_bytes) {
+                                  int64_t segs, bool fine) {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
@@ -1178,11 +1179,12 @@ static int64_t choose_super_tiles(int64_t nst, int64_t n_items, int64_t Hkv, int
   // does not: a batch-1 32k context over 28 layers then runs as one full round
   // instead of ~1.9 (+3 % measured).
   if (units * splits(nst) > round) return units * splits(2 * nst) <= round ? 2 * nst : nst;
+  if (!fine) return nst;
   const int64_t n_super = ceil_div(max_tq, decode_mfma_split_tokens(bits, 1));
   int64_t best = nst, best_cost = INT64_MAX;
   for (int64_t n = nst; n >= 1; --n) {
     const int64_t sp = ceil_div(n_super, n), groups = units * splits(n);
-    if (sp == 0 || groups > round || decode_mfma_workspace_bytes(n_items, Hkv, splits(n)) > workspace_bytes) break;
+    if (sp == 0 || groups > min(round, kWgPerCu * kCus)) break;  // kCus: what the workspace is sized for
     const int64_t tile = groups <= cus ? 15 : groups <= 2 * cus ? 20 : 30;
     const int64_t cost = ceil_div(n_super, sp) * tile + segs * splits(n);
     if (cost < best_cost) best = n, best_cost = cost;
@@ -1193,8 +1195,8 @@ static int64_t choose_super_tiles(int64_t nst, int64_t n_items, int64_t Hkv, int
 int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single, int64_t n_items, int bits,
                        int group_size, int64_t Hq, int64_t Hkv, int64_t Lq, int q_dtype, int res_dtype,
                        int out_dtype, float sm_scale, int64_t max_tq, int64_t max_tr, int64_t nst, int64_t segs,
-                       void *workspace, int64_t workspace_bytes, hipStream_t stream) {
-  nst = choose_super_tiles(nst, n_items, Hkv, bits, max_tq, max_tr, segs, workspace_bytes);
+                       bool fine, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
+  nst = choose_super_tiles(nst, n_items, Hkv, bits, max_tq, max_tr, segs, fine);
   const int64_t s_tok = decode_mfma_split_tokens(bits, nst);
   MfmaParams p{};
   p.Hq = Hq; p.Hkv = Hkv; p.Lq = Lq; p.group = Hq / Hkv; p.rows = p.group * Lq;

@@ -3,9 +3,11 @@
 KiviDecodeBatch fixes, once, a device table of (packed segment, residual,
 query, output) items -- e.g. every (layer, sequence) of a decode step -- plus
 the outputs and the split-K workspace.  run() then enqueues a single
-uc_kivi_attn_decode_batch launch (and its LSE combine) and allocates nothing,
+uc_kivi_attn_decode_fine launch (and its LSE combine) and allocates nothing,
 so it can sit in a tight decode loop or a captured HIP graph.  Callers update
-the query tensors in place between steps.
+the query tensors in place between steps.  The split size follows from the
+whole launch, so a segment's last bits may differ from those of a launch of
+another size.
 
 The device tables hold raw pointers, so both classes check every pointer on
 the host when they build a table (device, the token-major packed layout,
@@ -150,7 +152,7 @@ class KiviDecodeBatch:
         lq, hq, d = self.shape
         first = self.caches[0]
         nat.call(
-            "uc_kivi_attn_decode_batch", self.table.data_ptr(), len(self.caches), first.k_bits,
+            "uc_kivi_attn_decode_fine", None, self.table.data_ptr(), len(self.caches), 1, first.k_bits,
             first.group_size, hq, first.num_kv_heads, d, lq, nat.dtype_code(self.queries[0].dtype),
             nat.dtype_code(self.res_dtype), nat.dtype_code(self.out_dtype), self.sm_scale, self.max_tq,
             self.max_tr, self.workspace.data_ptr(), self.ws_bytes,
@@ -162,7 +164,7 @@ class MixedDecodeBatch:
     """Decode over groups of KV segments that share one query: each group is a
     list of PackedKIVICache segments and dense (key, value) [T, Hkv, D]
     segments (bf16 H2O / protected tokens) and is attended as one softmax over
-    all of them by a single uc_kivi_attn_decode_segments launch for every
+    all of them by a single uc_kivi_attn_decode_fine launch for every
     group -- the decode form of _run_fused_mixed_attention
     (adapters/bagel.py:1598-1858) without concatenating the segments.
 
@@ -419,7 +421,7 @@ class MixedDecodeBatch:
         self._guard.check("MixedDecodeBatch.run")
         lq, hq, d = self.shape
         nat.call(
-            "uc_kivi_attn_decode_segments", self.table.data_ptr(), self.n_items, self.segs, self.bits,
+            "uc_kivi_attn_decode_fine", None, self.table.data_ptr(), self.n_items, self.segs, self.bits,
             self.group_size, hq, self.kv_heads, d, lq, nat.dtype_code(self.queries[0].dtype),
             nat.dtype_code(self.res_dtype), nat.dtype_code(self.out_dtype), self.sm_scale, self.max_tq,
             self.max_tr, self.workspace.data_ptr(), self.ws_bytes,

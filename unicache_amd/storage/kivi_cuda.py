@@ -107,9 +107,9 @@ def _decode_summary(cache: "PackedKIVICache", query: torch.Tensor, *, include_re
     ws = nat.workspace(device, ws_bytes)
     res_dtype = cache.residual_key.dtype if tr else q.dtype
     nat.call(
-        "uc_kivi_attn_decode", item, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d, lq,
+        "uc_kivi_attn_decode_fine", item, None, 1, 1, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d, lq,
         nat.dtype_code(q.dtype), nat.dtype_code(res_dtype), nat.dtype_code(out_dtype),
-        1.0 / math.sqrt(d), ws.data_ptr(), ws_bytes, nat.stream(device),
+        1.0 / math.sqrt(d), 0, 0, ws.data_ptr(), ws_bytes, nat.stream(device),
     )
     return out, lse
 
@@ -207,17 +207,18 @@ def packed_summary_with_dense(
     if lq <= _max_decode_query_len(cache, hq):
         ws_bytes = nat.decode_preferred_workspace_bytes(1, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d,
                                                         lq, cache.quantized_tokens, tr)
-        entry = "uc_kivi_attn_decode"
-    else:
-        if d != 128 or cache.group_size not in (32, 64, 128) or (tr and dk.dtype not in (torch.bfloat16,
-                                                                                        torch.float16)):
-            raise ValueError("Mixed-segment attention needs head_dim 128, group 32/64/128 and 16-bit dense KV")
-        ws_bytes = 0  # the multi-query kernel needs no workspace
-        entry = "uc_kivi_attn_mq"
-    ws = nat.workspace(device, ws_bytes) if ws_bytes else None
-    nat.call(
-        entry, item, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d, lq, nat.dtype_code(q.dtype),
-        res_code, nat.dtype_code(q.dtype), 1.0 / math.sqrt(d), nat.ptr(ws), ws_bytes, nat.stream(device),
+        ws = nat.workspace(device, ws_bytes)
+        nat.call(
+            "uc_kivi_attn_decode_fine", item, None, 1, 1, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d,
+            lq, nat.dtype_code(q.dtype), res_code, nat.dtype_code(q.dtype), 1.0 / math.sqrt(d), 0, 0, ws.data_ptr(),
+            ws_bytes, nat.stream(device),
+        )
+        return out, lse
+    if d != 128 or cache.group_size not in (32, 64, 128) or (tr and dk.dtype not in (torch.bfloat16, torch.float16)):
+        raise ValueError("Mixed-segment attention needs head_dim 128, group 32/64/128 and 16-bit dense KV")
+    nat.call(  # no workspace
+        "uc_kivi_attn_mq", item, cache.k_bits, cache.group_size, hq, cache.num_kv_heads, d, lq,
+        nat.dtype_code(q.dtype), res_code, nat.dtype_code(q.dtype), 1.0 / math.sqrt(d), None, 0, nat.stream(device),
     )
     return out, lse
 
@@ -409,7 +410,7 @@ def packed_segments_summary(packed: list, query: torch.Tensor, dense: list,
     return out, lse
 
 
-DECODE_MAX_SEGMENTS = 8  # items one uc_kivi_attn_decode_segments_host call takes
+DECODE_MAX_SEGMENTS = 8  # items in host memory that one uc_kivi_attn_decode_fine call takes
 
 
 def decode_segments_supported(packed: list, query: torch.Tensor, dense: list) -> bool:
@@ -448,7 +449,7 @@ def decode_segments_summary(packed: list, query: torch.Tensor, dense: list) -> t
     and the dense (key, value) [T, Hkv, 128] parts `dense` -- any token and
     head strides, so an H2O segment's [Hkv, R, 128] tensors enter transposed,
     as views -- in one launch of the split-K decode kernels
-    (uc_kivi_attn_decode_segments_host): the segments are read where they lie,
+    (uc_kivi_attn_decode_fine): the segments are read where they lie,
     nothing is concatenated and no summaries are merged.  This is the decode
     form of _run_fused_mixed_attention (adapters/bagel.py:1598-1858).  Returns
     (out [Lq, Hq, 128] in the query dtype, lse [Hq, Lq])."""
@@ -492,9 +493,9 @@ def decode_segments_summary(packed: list, query: torch.Tensor, dense: list) -> t
         max_tr = max(max_tr, t)
     ws_bytes = nat.decode_preferred_workspace_bytes(n, first.k_bits, first.group_size, hq, hkv, d, lq, max_tq, max_tr)
     workspace = nat.workspace(device, ws_bytes)
-    nat.call("uc_kivi_attn_decode_segments_host", items, n, first.k_bits, first.group_size, hq, hkv, d, lq,
+    nat.call("uc_kivi_attn_decode_fine", items, None, n, n, first.k_bits, first.group_size, hq, hkv, d, lq,
              nat.dtype_code(q.dtype), nat.dtype_code(res_dtype), nat.dtype_code(q.dtype), 1.0 / math.sqrt(d),
-             workspace.data_ptr(), ws_bytes, nat.stream(device))
+             0, 0, workspace.data_ptr(), ws_bytes, nat.stream(device))
     return out, lse
 
 
@@ -630,15 +631,15 @@ def dense_attention_summary(
     bits, group = 2, 32  # no packed tokens: only the dense (residual) part is read
     if lq <= max(1, 16 // (hq // hkv)):
         ws_bytes = nat.decode_preferred_workspace_bytes(1, bits, group, hq, hkv, d, lq, 0, tokens)
-        entry = "uc_kivi_attn_decode"
-    else:
-        if d != 128:
-            raise ValueError("Dense attention over more than 16 query rows per KV head needs head_dim 128")
-        ws_bytes = 0  # the multi-query kernel needs no workspace
-        entry = "uc_kivi_attn_mq"
-    ws = nat.workspace(device, ws_bytes) if ws_bytes else None
-    nat.call(entry, item, bits, group, hq, hkv, d, lq, nat.dtype_code(q.dtype), nat.dtype_code(dk.dtype),
-             nat.dtype_code(q.dtype), 1.0 / math.sqrt(d), nat.ptr(ws), ws_bytes, nat.stream(device))
+        ws = nat.workspace(device, ws_bytes)
+        nat.call("uc_kivi_attn_decode_fine", item, None, 1, 1, bits, group, hq, hkv, d, lq, nat.dtype_code(q.dtype),
+                 nat.dtype_code(dk.dtype), nat.dtype_code(q.dtype), 1.0 / math.sqrt(d), 0, 0, ws.data_ptr(), ws_bytes,
+                 nat.stream(device))
+        return out, lse
+    if d != 128:
+        raise ValueError("Dense attention over more than 16 query rows per KV head needs head_dim 128")
+    nat.call("uc_kivi_attn_mq", item, bits, group, hq, hkv, d, lq, nat.dtype_code(q.dtype), nat.dtype_code(dk.dtype),
+             nat.dtype_code(q.dtype), 1.0 / math.sqrt(d), None, 0, nat.stream(device))  # no workspace
     return out, lse
 
 

@@ -709,7 +709,7 @@ int64_t uc_kivi_decode_workspace_bytes(int64_t n_items, int bits, int group_size
 
 /*
  * The same for uc_kivi_attn_decode_fine: at least
- * uc_kivi_decode_workspace_bytes and at most about 3.3 MB more.
+ * uc_kivi_decode_workspace_bytes and at most about 6.4 MB more.
  */
 int64_t uc_kivi_decode_preferred_workspace_bytes(int64_t n_items, int bits, int group_size, int64_t heads_q,
                                                  int64_t heads_kv, int64_t head_dim, int64_t query_len,

@@ -244,6 +244,53 @@ def test_decode_results_do_not_depend_on_workspace(device, bits, group, tokens, 
         summary("uc_kivi_attn_decode_fine", 4)
 
 
+@pytest.mark.parametrize("bits,group,hq,lq,lengths", [(2, 32, 28, 1, (2048,)), (2, 64, 28, 2, (2048, 1024, 256)),
+                                                      (4, 64, 16, 1, (1024,)), (4, 128, 32, 2, (8192,) * 4),
+                                                      (2, 32, 12, 1, (32768, 512)), (2, 32, 32, 1, (8192,) * 8)])
+def test_finer_splits_hand_over_fp32_partials(device, bits, group, hq, lq, lengths):
+    # zero keys weigh all tokens alike and V alternates between two fp16 values
+    # whose mean is none: every product and sum is exact in fp32, an fp16 partial
+    # is off by 2^-11.  3 to 16 query rows per KV head, 1 to 128 super-tiles
+    from unicache_amd.storage.decode import KiviDecodeBatch
+
+    caches = []
+    for tokens in lengths:
+        value = torch.ones(tokens, 4, 128, dtype=torch.float16, device=device)
+        value[1::2] += 2.0 ** -10
+        caches.append(PackedKIVICache.from_dense(
+            torch.zeros_like(value), value, logical_token_ids=torch.arange(tokens), token_type_id=3, k_bits=bits,
+            v_bits=bits, group_size=group, residual_length=0, backend="cuda"))
+    q = [queries(lq, heads=hq, seed=160 + i, dtype=torch.float16).to(device) for i in range(len(caches))]
+    args = (len(caches), bits, group, hq, 4, 128, lq, max(lengths), 0)
+    assert nat.decode_preferred_workspace_bytes(*args) > nat.decode_workspace_bytes(*args)
+    batch = KiviDecodeBatch(caches, q, out_dtype=torch.float32)
+    batch.run()
+    for i, tokens in enumerate(lengths):
+        # the normalisations and the weighted sum: a few fp32 roundings each
+        assert float((batch.outputs[i] - (1 + 2.0 ** -11)).abs().max()) <= 2.0 ** -20
+        assert float((batch.lses[i] - math.log(tokens)).abs().max()) <= 1e-5
+    one = KiviDecodeBatch(caches[:1], q[:1])
+    one.run()
+    out, lse = packed_kivi_attention_summary(caches[0], q[0])  # the item in the kernel arguments
+    assert torch.equal(out, one.outputs[0]) and torch.equal(lse, one.lses[0])
+
+
+def test_decode_combine_of_many_splits(device):
+    # one packed segment and 7 dense ones of up to 13 splits at 4 query rows per
+    # KV head: 112 splits, the 16 parts a combine block takes at most
+    from unicache_amd.storage.kivi_cuda import decode_segments_summary
+
+    cache, seg = _pair(64, 170, 2, 32, 0, device, heads=8)
+    parts = [kv_pair(3300 - 50 * i, heads=8, seed=171 + i) for i in range(7)]
+    q = queries(1, heads=32, seed=180)
+    out, lse = decode_segments_summary([cache], q.to(device), [(k.to(device), v.to(device)) for k, v in parts])
+    key, value = K.dequantize(seg, "fp32")
+    eo, el = A.attention_summary(f32(q), np.concatenate([key] + [f32(k) for k, _ in parts]),
+                                 np.concatenate([value] + [f32(v) for _, v in parts]))
+    assert_close(f32(out), eo, what="out")
+    assert_close(f32(lse), el, max_abs=1e-2, mean_abs=1e-3, what="lse")
+
+
 def test_decode_is_deterministic(device):
     cache, _ = _pair(4096, 11, 2, 32, 128, device)
     q = queries(1, seed=2).to(device)

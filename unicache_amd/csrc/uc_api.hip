@@ -87,8 +87,9 @@ extern "C" int64_t uc_kivi_decode_preferred_workspace_bytes(int64_t n_items, int
                                                             int64_t max_residual_tokens) {
   const int64_t least = uc_kivi_decode_workspace_bytes(n_items, bits, group_size, heads_q, heads_kv, head_dim,
                                                        query_len, max_quantized_tokens, max_residual_tokens);
-  if (least < 0 || !uc::decode_mfma_supported(bits, group_size, head_dim, (heads_q / heads_kv) * query_len))
-    return least;
-  return uc::decode_mfma_preferred_workspace_bytes(n_items, heads_kv, bits, max_quantized_tokens,
+  if (least < 0) return least;
+  const int64_t rows = (heads_q / heads_kv) * query_len;
+  if (!uc::decode_mfma_supported(bits, group_size, head_dim, rows)) return least;
+  return uc::decode_mfma_preferred_workspace_bytes(n_items, heads_kv, rows, bits, max_quantized_tokens,
                                                    max_residual_tokens);
 }

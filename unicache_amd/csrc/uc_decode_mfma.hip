@@ -34,12 +34,15 @@
 // B' products, logit FMAs and exponentials are halved; the two halves merge
 // by a lane exchange at the end of the split.
 //
-// Each split writes a normalised fp16 partial of its query rows with its
-// (max, sum); decode_mfma_combine merges the splits by log-sum-exp.
+// Each split writes a normalised partial of its query rows with its (max, sum);
+// decode_mfma_combine merges the splits by log-sum-exp.  Splits of kDecodeMfmaNst
+// super-tiles or more write fp16.  Finer ones write fp32: what they hand over
+// would have stayed in the fp32 accumulators of a longer split.
 #include "uc_common.h"
 #include "uc_decode.h"
 #include "uc_mfma.h"
 
+#include <type_traits>
 
 namespace uc {
 namespace {
@@ -160,7 +163,8 @@ struct MfmaParams {
   int64_t super_tokens;                      // tokens per super-tile (16 key words)
   int xcd_grouped;                           // splits of a unit on one XCD (see the kernel)
   float scale_log2;
-  _Float16 *ws_o;  // [items * Hkv * splits][16][128] normalised partial outputs
+  void *ws_o;      // normalised partial outputs: [items * Hkv * splits][16][128] fp16, or [..][o_rows][128] fp32
+  int o_rows;
   float *ws_ml;    // [items * Hkv * splits][16][2] (max in log2 units, sum)
   int qd, rd, od;
 };
@@ -860,7 +864,7 @@ __device__ __forceinline__ void residual_split(const _Float16 (*sq)[kQPad], cons
 }
 
 // ------------------------------------------------------------------ kernel --
-template <int BITS, int G, int RD, bool TABLE, bool FOLD>
+template <int BITS, int G, int RD, bool TABLE, bool FOLD, bool F32>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) void decode_mfma_kernel(
     const uc_kivi_item *items, ArgItems ai, MfmaParams p) {
   __shared__ __align__(16) DecShared<BITS, G> sh;
@@ -947,7 +951,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
   __syncthreads();
   if (wave == 0) {
     const int64_t slot = (item * p.Hkv + h) * p.splits_total + split;
-    _Float16 *po = p.ws_o + slot * 16 * kD;
+    typedef typename std::conditional<F32, float, _Float16>::type Part;
+    Part *po = static_cast<Part *>(p.ws_o) + slot * (F32 ? p.o_rows : 16) * kD;
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
     if (n < p.rows) {  // rows past the query rows are never read: not written
 #pragma unroll
@@ -955,7 +960,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
         f4 s = st.o[b] * mine;
 #pragma unroll
         for (int w = 0; w < kWaves - 1; ++w) s += *reinterpret_cast<const f4 *>(&sh.mrg.o[w][n][16 * b + 4 * kap]);
-        *reinterpret_cast<h4 *>(&po[n * kD + 16 * b + 4 * kap]) = cvt4(s * inv);
+        if constexpr (F32)
+          *reinterpret_cast<f4 *>(&po[n * kD + 16 * b + 4 * kap]) = s * inv;
+        else
+          *reinterpret_cast<h4 *>(&po[n * kD + 16 * b + 4 * kap]) = cvt4(s * inv);
       }
     }
     if (kap == 0) {
@@ -967,56 +975,69 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
 
 // Merge the split partials of one (query group, KV head) -- every split of the
 // p.segs items that share the query.  Thread (row = t / 16, c = t % 16) of a
-// part owns channels 8c .. 8c + 7 of one query row, so a row's 16 threads read
-// each partial row as one contiguous 256-byte run; a part has only the threads
-// of the query rows (rounded to whole waves).  The splits are dealt to
-// `parts` (1, 2, 4 or 8) parts of the block in contiguous runs; a part takes its
-// run in rounds of kCombineRound, every load of a round issued before any
-// arithmetic, with an online (M, L): a round that raises the maximum rescales
-// the sums first.  The parts then merge through LDS, part 0 writes the output
-// and the LSE of the group's first item.  Splits without work wrote (-inf, 0)
-// and no partial: their weight is 0 and their partial is not read.
+// part owns 16 bytes of one query row's partial: channels 8c .. 8c + 7 of fp16
+// partials, 4c .. 4c + 3 of the block's half of the channels of fp32 ones (two
+// blocks, so as many loads are in flight with the same registers).  A row's 16
+// threads read each partial row as one contiguous 256-byte run; a part has only
+// the threads of the query rows (rounded to whole waves).  The splits are dealt
+// to `parts` (a power of two up to 16: kCombineMaxThreads / the threads of a
+// part) parts of the block in contiguous runs; a part takes its run in rounds
+// of kCombineRound, every load of a round issued before any arithmetic, with an
+// online (M, L): a round that raises the maximum rescales the sums first.  The
+// parts then merge through LDS, part 0 writes the output and the LSE of the
+// group's first item.  Splits without work wrote (-inf, 0) and no partial:
+// their weight is 0 and their partial is not read.
 constexpr int kCombineRound = 16;
 constexpr int kCombineRun = 12;  // splits a part takes before the launch adds parts
 constexpr int kCombineMaxThreads = 1024;
 
-// Eight channels of output element `idx` on, from fp32 (one 16-byte store for
-// 16-bit outputs).
-__device__ __forceinline__ void store_out8(void *out, int64_t idx, const float *v, int od) {
+// N (4 or 8) channels of output element `idx` on, from fp32 (one 2N-byte store
+// for 16-bit outputs).
+template <int N>
+__device__ __forceinline__ void store_out(void *out, int64_t idx, const float *v, int od) {
   if (od == UC_FP32) {
     float4 *o = reinterpret_cast<float4 *>(static_cast<float *>(out) + idx);
-    o[0] = make_float4(v[0], v[1], v[2], v[3]);
-    o[1] = make_float4(v[4], v[5], v[6], v[7]);
+#pragma unroll
+    for (int k = 0; k < N / 4; ++k) o[k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
     return;
   }
-  uint32_t w[4];
+  uint32_t w[N / 2];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < N / 2; ++k) {
     const uint32_t lo = od == UC_BF16 ? f32_to_bf16_bits(v[2 * k]) : f32_to_f16_bits(v[2 * k]);
     const uint32_t hi = od == UC_BF16 ? f32_to_bf16_bits(v[2 * k + 1]) : f32_to_f16_bits(v[2 * k + 1]);
     w[k] = lo | (hi << 16);
   }
-  *reinterpret_cast<uint4 *>(static_cast<uint16_t *>(out) + idx) = make_uint4(w[0], w[1], w[2], w[3]);
+  uint16_t *o = static_cast<uint16_t *>(out) + idx;
+  if constexpr (N == 8)
+    *reinterpret_cast<uint4 *>(o) = make_uint4(w[0], w[1], w[2], w[3]);
+  else
+    *reinterpret_cast<uint2 *>(o) = make_uint2(w[0], w[1]);
 }
 
-template <bool TABLE>
+// Channels one thread of the combine owns.
+template <bool F32>
+constexpr int kCombineChannels = F32 ? 4 : 8;
+
+template <bool TABLE, bool F32>
 __global__ __launch_bounds__(kCombineMaxThreads) void decode_mfma_combine(const uc_kivi_item *items, ArgItems ai,
                                                                           MfmaParams p, int parts) {
-  extern __shared__ float red[];  // per thread of parts 1..: M, L, 8 sums (10 floats)
+  constexpr int C = kCombineChannels<F32>;
+  extern __shared__ float red[];  // per thread of parts 1..: M, L, C sums
   const int64_t first = blockIdx.x * p.segs;
   const int64_t h = blockIdx.y;
   const int span = int(blockDim.x) / parts;  // threads per part (whole waves)
   const int part = int(threadIdx.x) / span, t = int(threadIdx.x) % span;
-  const int r = t >> 4, c8 = (t & 15) * 8;
+  const int r = t >> 4, c0 = (int(blockIdx.z) * 16 + (t & 15)) * C;
   const bool active = r < p.rows;
   const int splits = int(p.splits_total), nflat = int(p.segs) * splits;
   const int run = (nflat + parts - 1) / parts, f_lo = part * run, f_hi = min(nflat, f_lo + run);
   // (segment, split) f -> workspace slot: segment f / splits of the group
   auto slot = [&](int f) { return ((first + f / splits) * p.Hkv + h) * p.splits_total + f % splits; };
   float M = kNegInf, L = 0.0f;
-  float acc[8];
+  float acc[C];
 #pragma unroll
-  for (int c = 0; c < 8; ++c) acc[c] = 0.0f;
+  for (int c = 0; c < C; ++c) acc[c] = 0.0f;
   for (int f0 = f_lo; active && f0 < f_hi; f0 += kCombineRound) {
     float2 ml[kCombineRound];
     uint4 v[kCombineRound];
@@ -1025,7 +1046,10 @@ __global__ __launch_bounds__(kCombineMaxThreads) void decode_mfma_combine(const 
       if (f0 + u < f_hi) {
         const int64_t sl = slot(f0 + u);
         ml[u] = *reinterpret_cast<const float2 *>(p.ws_ml + (sl * 16 + r) * 2);
-        v[u] = *reinterpret_cast<const uint4 *>(p.ws_o + (sl * 16 + r) * kD + c8);
+        if constexpr (F32)
+          v[u] = *reinterpret_cast<const uint4 *>(static_cast<const float *>(p.ws_o) + (sl * p.o_rows + r) * kD + c0);
+        else
+          v[u] = *reinterpret_cast<const uint4 *>(static_cast<const _Float16 *>(p.ws_o) + (sl * 16 + r) * kD + c0);
       } else {
         ml[u] = make_float2(kNegInf, 0.0f);
       }
@@ -1038,7 +1062,7 @@ __global__ __launch_bounds__(kCombineMaxThreads) void decode_mfma_combine(const 
       const float sc = M == kNegInf ? 0.0f : exp2f(M - mr);
       L *= sc;
 #pragma unroll
-      for (int c = 0; c < 8; ++c) acc[c] *= sc;
+      for (int c = 0; c < C; ++c) acc[c] *= sc;
       M = mr;
     }
 #pragma unroll
@@ -1049,30 +1073,34 @@ __global__ __launch_bounds__(kCombineMaxThreads) void decode_mfma_combine(const 
       const uint32_t wd[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        acc[2 * e] = fmaf(f16_bits_to_f32(uint16_t(wd[e] & 0xffffu)), w, acc[2 * e]);
-        acc[2 * e + 1] = fmaf(f16_bits_to_f32(uint16_t(wd[e] >> 16)), w, acc[2 * e + 1]);
+        if constexpr (F32) {
+          acc[e] = fmaf(__uint_as_float(wd[e]), w, acc[e]);
+        } else {
+          acc[2 * e] = fmaf(f16_bits_to_f32(uint16_t(wd[e] & 0xffffu)), w, acc[2 * e]);
+          acc[2 * e + 1] = fmaf(f16_bits_to_f32(uint16_t(wd[e] >> 16)), w, acc[2 * e + 1]);
+        }
       }
     }
   }
   if (parts > 1) {  // uniform
     if (part > 0) {
-      float *e = red + (threadIdx.x - span) * 10;
+      float *e = red + (threadIdx.x - span) * (2 + C);
       e[0] = M;
       e[1] = L;
 #pragma unroll
-      for (int c = 0; c < 8; ++c) e[2 + c] = acc[c];
+      for (int c = 0; c < C; ++c) e[2 + c] = acc[c];
     }
     __syncthreads();
     if (part > 0) return;
     for (int q = 1; q < parts; ++q) {
-      const float *e = red + ((q - 1) * span + t) * 10;
+      const float *e = red + ((q - 1) * span + t) * (2 + C);
       const float m2 = e[0], l2 = e[1];
       if (!(l2 > 0.0f)) continue;
       const float mn = fmaxf(M, m2);
       const float s1 = M == kNegInf ? 0.0f : exp2f(M - mn), s2 = exp2f(m2 - mn);
       L = L * s1 + l2 * s2;
 #pragma unroll
-      for (int c = 0; c < 8; ++c) acc[c] = acc[c] * s1 + e[2 + c] * s2;
+      for (int c = 0; c < C; ++c) acc[c] = acc[c] * s1 + e[2 + c] * s2;
       M = mn;
     }
   }
@@ -1080,10 +1108,10 @@ __global__ __launch_bounds__(kCombineMaxThreads) void decode_mfma_combine(const 
   const uc_kivi_item it = TABLE ? items[first] : ai.v[first];
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
 #pragma unroll
-  for (int c = 0; c < 8; ++c) acc[c] *= inv;
+  for (int c = 0; c < C; ++c) acc[c] *= inv;
   const int64_t g = r / p.Lq, i = r % p.Lq;
-  if (c8 == 0 && it.lse != nullptr) it.lse[(h * p.group + g) * p.Lq + i] = L > 0.0f ? (M + log2f(L)) * kLn2 : kNegInf;
-  store_out8(it.out, (i * p.Hq + h * p.group + g) * kD + c8, acc, p.od);
+  if (c0 == 0 && it.lse != nullptr) it.lse[(h * p.group + g) * p.Lq + i] = L > 0.0f ? (M + log2f(L)) * kLn2 : kNegInf;
+  store_out<C>(it.out, (i * p.Hq + h * p.group + g) * kD + c0, acc, p.od);
 }
 
 }  // namespace
@@ -1099,14 +1127,24 @@ int64_t decode_mfma_num_splits(int bits, int64_t nst, int64_t max_tq, int64_t ma
   return ceil_div(max_tq, decode_mfma_split_tokens(bits, nst)) + ceil_div(max_tr, decode_mfma_res_split_tokens(max_tr));
 }
 
-int64_t decode_mfma_preferred_workspace_bytes(int64_t n_items, int64_t heads_kv, int bits, int64_t max_tq,
-                                              int64_t max_tr) {
+// Query rows an fp32 partial has room for: eight fp32 rows fit where sixteen
+// fp16 ones do.
+static int64_t fp32_partial_rows(int64_t rows) { return rows <= 8 ? 8 : 16; }
+
+// Bytes of one split's partial with its (max, sum) rows.
+static int64_t fp16_slot_bytes() { return 16 * (kD * int64_t(sizeof(_Float16)) + 2 * int64_t(sizeof(float))); }
+static int64_t fp32_slot_bytes(int64_t rows) {
+  return (fp32_partial_rows(rows) * kD + 16 * 2) * int64_t(sizeof(float));
+}
+
+int64_t decode_mfma_preferred_workspace_bytes(int64_t n_items, int64_t heads_kv, int64_t rows, int bits,
+                                              int64_t max_tq, int64_t max_tr) {
   const int64_t units = n_items * heads_kv;
   const int64_t least = decode_mfma_workspace_bytes(n_items, heads_kv,
                                                     decode_mfma_num_splits(bits, kDecodeMfmaNst, max_tq, max_tr));
   // finer splits (choose_super_tiles) stay within one round of workgroup slots
   const int64_t fine = min(units * decode_mfma_num_splits(bits, 1, max_tq, max_tr), kWgPerCu * kCus);
-  return max(least, decode_mfma_workspace_bytes(1, 1, fine));
+  return max(least, fine * fp32_slot_bytes(rows));
 }
 
 bool decode_mfma_supported(int bits, int group, int64_t D, int64_t rows) {
@@ -1114,43 +1152,50 @@ bool decode_mfma_supported(int bits, int group, int64_t D, int64_t rows) {
 }
 
 int64_t decode_mfma_workspace_bytes(int64_t n_items, int64_t heads_kv, int64_t splits) {
-  const int64_t slots = n_items * heads_kv * splits;
-  return slots * 16 * kD * int64_t(sizeof(_Float16)) + slots * 16 * 2 * int64_t(sizeof(float));
+  return n_items * heads_kv * splits * fp16_slot_bytes();
 }
 
 // The column-folded packed path: 2-bit codes, 32-token groups, <= 8 query rows.
 template <int BITS, int G>
 constexpr bool kFoldable = BITS == 2 && G == 32;
 
+// What a launch of decode_mfma_kernel takes beside its types.
+struct DecodeLaunch {
+  bool table, f32;
+  dim3 grid;
+  hipStream_t stream;
+  const uc_kivi_item *items_dev;
+  ArgItems one;
+  MfmaParams p;
+};
+
+template <int BITS, int G, int RD, bool FOLD, bool F32>
+static void launch_typed(const DecodeLaunch &l) {
+  if (l.table)
+    hipLaunchKernelGGL((decode_mfma_kernel<BITS, G, RD, true, FOLD, F32>), l.grid, dim3(kThreads), 0, l.stream,
+                       l.items_dev, l.one, l.p);
+  else
+    hipLaunchKernelGGL((decode_mfma_kernel<BITS, G, RD, false, FOLD, F32>), l.grid, dim3(kThreads), 0, l.stream,
+                       l.items_dev, l.one, l.p);
+}
+
 template <int BITS, int G, int RD>
-static void launch_typed(bool table, dim3 grid, hipStream_t stream, const uc_kivi_item *items_dev,
-                         const ArgItems &one, const MfmaParams &p) {
+static void launch_fold(const DecodeLaunch &l) {
   if constexpr (kFoldable<BITS, G>) {
-    if (p.rows <= 8) {
-      if (table)
-        hipLaunchKernelGGL((decode_mfma_kernel<BITS, G, RD, true, true>), grid, dim3(kThreads), 0, stream, items_dev,
-                           one, p);
-      else
-        hipLaunchKernelGGL((decode_mfma_kernel<BITS, G, RD, false, true>), grid, dim3(kThreads), 0, stream, items_dev,
-                           one, p);
+    if (l.p.rows <= 8) {
+      if (l.f32) launch_typed<BITS, G, RD, true, true>(l);
+      else launch_typed<BITS, G, RD, true, false>(l);
       return;
     }
   }
-  if (table)
-    hipLaunchKernelGGL((decode_mfma_kernel<BITS, G, RD, true, false>), grid, dim3(kThreads), 0, stream, items_dev,
-                       one, p);
-  else
-    hipLaunchKernelGGL((decode_mfma_kernel<BITS, G, RD, false, false>), grid, dim3(kThreads), 0, stream, items_dev,
-                       one, p);
+  if (l.f32) launch_typed<BITS, G, RD, false, true>(l);
+  else launch_typed<BITS, G, RD, false, false>(l);
 }
 
 template <int BITS, int G>
-static void launch_group(bool table, int rd, dim3 grid, hipStream_t stream, const uc_kivi_item *items_dev,
-                         const ArgItems &one, const MfmaParams &p) {
-  if (rd == UC_FP16)
-    launch_typed<BITS, G, UC_FP16>(table, grid, stream, items_dev, one, p);
-  else
-    launch_typed<BITS, G, UC_BF16>(table, grid, stream, items_dev, one, p);
+static void launch_group(const DecodeLaunch &l) {
+  if (l.p.rd == UC_FP16) launch_fold<BITS, G, UC_FP16>(l);
+  else launch_fold<BITS, G, UC_BF16>(l);
 }
 
 // Super-tiles per packed split of a launch.  `nst` per split is the right size
@@ -1196,6 +1241,7 @@ int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single
                        int group_size, int64_t Hq, int64_t Hkv, int64_t Lq, int q_dtype, int res_dtype,
                        int out_dtype, float sm_scale, int64_t max_tq, int64_t max_tr, int64_t nst, int64_t segs,
                        bool fine, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
+  const int64_t usual = nst;
   nst = choose_super_tiles(nst, n_items, Hkv, bits, max_tq, max_tr, segs, fine);
   const int64_t s_tok = decode_mfma_split_tokens(bits, nst);
   MfmaParams p{};
@@ -1212,16 +1258,19 @@ int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single
   UC_REQUIRE(max_tq * (kD / 8) * 4 < (int64_t(1) << 31) && max_tr * Hkv * kD * 2 < (int64_t(1) << 31),
              "decode: segment too long for 32-bit buffer offsets (%lld packed, %lld residual tokens)",
              (long long)max_tq, (long long)max_tr);
-  const int64_t need = decode_mfma_workspace_bytes(n_items, Hkv, p.splits_total);
+  const bool f32 = nst < usual;
+  p.o_rows = static_cast<int>(fp32_partial_rows(p.rows));
+  const int64_t slots = n_items * Hkv * p.splits_total;
+  const int64_t need = slots * (f32 ? fp32_slot_bytes(p.rows) : fp16_slot_bytes());
   UC_REQUIRE(workspace != nullptr && workspace_bytes >= need, "decode: workspace too small (%lld < %lld bytes)",
              (long long)workspace_bytes, (long long)need);
-  const int64_t slots = n_items * Hkv * p.splits_total;
-  p.ws_o = static_cast<_Float16 *>(workspace);
-  p.ws_ml = reinterpret_cast<float *>(static_cast<char *>(workspace) + slots * 16 * kD * sizeof(_Float16));
+  p.ws_o = workspace;
+  p.ws_ml = reinterpret_cast<float *>(static_cast<char *>(workspace) + need) - slots * 16 * 2;
   const bool table = items_dev != nullptr;
   UC_REQUIRE(table || (single != nullptr && n_items <= kArgItems), "decode: at most %d items from host memory",
              kArgItems);
-  ArgItems one{};
+  DecodeLaunch l{};
+  ArgItems &one = l.one;
   if (!table)
     for (int64_t i = 0; i < n_items; ++i) one.v[i] = single[i];
   p.units = n_items * Hkv;
@@ -1229,15 +1278,20 @@ int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single
   p.xcd_grouped = p.units >= 4 * kXcds;  // at most one unit of imbalance per XCD in four
   const int64_t n_groups = (p.xcd_grouped ? ceil_div(p.units, int64_t(kXcds)) * kXcds : p.units) * p.splits_total;
   UC_REQUIRE(n_groups < (int64_t(1) << 31), "decode: grid too large (%lld workgroups)", (long long)n_groups);
-  const dim3 grid(static_cast<unsigned>(n_groups));
+  l.table = table;
+  l.f32 = f32;
+  l.grid = dim3(static_cast<unsigned>(n_groups));
+  l.stream = stream;
+  l.items_dev = items_dev;
+  l.p = p;
   if (bits == 2) {
-    if (group_size == 32) launch_group<2, 32>(table, res_dtype, grid, stream, items_dev, one, p);
-    else if (group_size == 64) launch_group<2, 64>(table, res_dtype, grid, stream, items_dev, one, p);
-    else launch_group<2, 128>(table, res_dtype, grid, stream, items_dev, one, p);
+    if (group_size == 32) launch_group<2, 32>(l);
+    else if (group_size == 64) launch_group<2, 64>(l);
+    else launch_group<2, 128>(l);
   } else {
-    if (group_size == 32) launch_group<4, 32>(table, res_dtype, grid, stream, items_dev, one, p);
-    else if (group_size == 64) launch_group<4, 64>(table, res_dtype, grid, stream, items_dev, one, p);
-    else launch_group<4, 128>(table, res_dtype, grid, stream, items_dev, one, p);
+    if (group_size == 32) launch_group<4, 32>(l);
+    else if (group_size == 64) launch_group<4, 64>(l);
+    else launch_group<4, 128>(l);
   }
   int rc = check_launch("decode (MFMA)");
   if (rc != UC_OK) return rc;
@@ -1249,13 +1303,18 @@ int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single
   const int64_t nflat = segs * p.splits_total, span = ceil_div(p.rows * 16, int64_t(kWave)) * kWave;
   int parts = 1;
   while (nflat > kCombineRun * parts && 2 * parts * span <= kCombineMaxThreads) parts *= 2;
-  const dim3 cgrid(static_cast<unsigned>(n_items / segs), static_cast<unsigned>(Hkv));
-  const dim3 cblock(static_cast<unsigned>(parts * span));
-  const size_t lds = size_t(cblock.x / parts) * (parts - 1) * 10 * sizeof(float);
-  if (table)
-    hipLaunchKernelGGL((decode_mfma_combine<true>), cgrid, cblock, lds, stream, items_dev, one, p, parts);
-  else
-    hipLaunchKernelGGL((decode_mfma_combine<false>), cgrid, cblock, lds, stream, items_dev, one, p, parts);
+  const auto combine = [&](auto f32_tag) {
+    constexpr bool F32 = decltype(f32_tag)::value;
+    const dim3 cgrid(static_cast<unsigned>(n_items / segs), static_cast<unsigned>(Hkv), F32 ? 2 : 1);
+    const dim3 cblock(static_cast<unsigned>(parts * span));
+    const size_t lds = size_t(span) * (parts - 1) * (2 + kCombineChannels<F32>) * sizeof(float);
+    if (table)
+      hipLaunchKernelGGL((decode_mfma_combine<true, F32>), cgrid, cblock, lds, stream, items_dev, one, p, parts);
+    else
+      hipLaunchKernelGGL((decode_mfma_combine<false, F32>), cgrid, cblock, lds, stream, items_dev, one, p, parts);
+  };
+  if (f32) combine(std::true_type{});
+  else combine(std::false_type{});
   return check_launch("decode (MFMA combine)");
 }
 

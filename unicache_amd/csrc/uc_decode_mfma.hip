@@ -42,6 +42,7 @@
 #include "uc_decode.h"
 #include "uc_mfma.h"
 
+#include <atomic>
 #include <type_traits>
 
 namespace uc {
@@ -164,9 +165,9 @@ struct MfmaParams {
   int xcd_grouped;                           // splits of a unit on one XCD (see the kernel)
   float scale_log2;
   void *ws_o;      // normalised partial outputs: [items * Hkv * splits][16][128] fp16, or [..][o_rows][128] fp32
-  int o_rows;
   float *ws_ml;    // [items * Hkv * splits][16][2] (max in log2 units, sum)
   int qd, rd, od;
+  int o_rows;      // rows of an fp32 partial
 };
 
 // Whether split `split` of an item with tq packed and tr residual tokens has
@@ -988,7 +989,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
 // group's first item.  Splits without work wrote (-inf, 0) and no partial:
 // their weight is 0 and their partial is not read.
 constexpr int kCombineRound = 16;
-constexpr int kCombineRun = 12;  // splits a part takes before the launch adds parts
 constexpr int kCombineMaxThreads = 1024;
 
 // N (4 or 8) channels of output element `idx` on, from fp32 (one 2N-byte store
@@ -1198,40 +1198,70 @@ static void launch_group(const DecodeLaunch &l) {
   else launch_fold<BITS, G, UC_BF16>(l);
 }
 
+// CUs of the current device (0 if unknown), asked for once per device.
+static int device_cus() {
+  constexpr int kMaxDevices = 64;
+  static std::atomic<int> known[kMaxDevices];
+  int dev = -1, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 0;
+  if (dev < kMaxDevices && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  if (dev < kMaxDevices) known[dev].store(cus, std::memory_order_relaxed);
+  return cus;
+}
+
+// Threads of a part of the combine, and the parts a block has room for.
+static int64_t combine_span(int64_t rows) { return ceil_div(rows * 16, int64_t(kWave)) * kWave; }
+static int64_t combine_max_parts(int64_t rows) {
+  int64_t parts = 1;
+  while (2 * parts * combine_span(rows) <= kCombineMaxThreads) parts *= 2;
+  return parts;
+}
+
 // Super-tiles per packed split of a launch.  `nst` per split is the right size
 // for launches of several rounds of workgroup slots (kWgPerCu per CU): there a
 // split's fixed cost counts.  A `fine` launch that does not fill one round is
 // bound by the longest split's serial chain instead, so it takes the split size
-// with the least estimated time: the chain's super-tiles at the measured 1.36, 1.8 or
-// 2.7 us each with 1, 2 or 3 workgroups on a CU (alone, a wave leaves half its
-// SIMD's issue slots idle; three waves fill them), plus 0.09 us per split that
-// the combine reads, in units of 0.09 us.  Measured, call to call: 8 sequences
-// of 2048 tokens at 2 bits 21.0 -> 12.6 us (1 super-tile), 8 x 8192 21.7 ->
-// 18.1 us (3), one 32768-token segment 21.9 -> 16.2 us (3; 18.6 with 2, 17.2
-// with 4), 8 x 8192 at 4 bits 21.8 -> 18.2 us (3); the estimate picked the
-// fastest or within 0.2 us of it on 15 shapes of 8 to 1024 super-tiles a unit.
+// with the least estimated time, in units of 0.09 us:
+//   - the chain's super-tiles with 1, 2 or 3 workgroups on a CU (alone, a wave
+//     leaves half its SIMD's issue slots idle; three waves fill them): about
+//     1.4, 1.8 and 2.7 us each at 2 bits and 1.3, 1.6 and 2.3 at 4, whose
+//     super-tile has half the tokens;
+//   - but no less than the dense splits take, which finer packed ones do not
+//     shorten: 0.036 us for 256 tokens of a KV head (176 such splits take 7 us,
+//     256 take 10.5);
+//   - and what a split costs the combine: 0.09 us, twice that for those past
+//     one round of loads of every part (64 splits with more than 8 query rows).
+// Call to call from 8 super-tiles a split: 8 sequences of 2048 tokens at 2 bits
+// 21.0 -> 12.6 us (1 super-tile), 8 x 8192 21.7 -> 18.1 us (3), one 32768-token
+// segment 21.9 -> 16.2 us (3), 8 x 8192 at 4 bits 21.8 -> 18.2 us (3).  Over 488
+// launches of 400 to 65536 tokens (1 to 224 items, 2 to 8 KV heads, with and
+// without dense segments) the choice is within 1 % of the fastest of the eight
+// sizes on average and within 4.5 % for 95 of 100.
 // The choice never looks at the size of the workspace, so results do not depend
 // on it.
-static int64_t choose_super_tiles(int64_t nst, int64_t n_items, int64_t Hkv, int bits, int64_t max_tq, int64_t max_tr,
-                                  int64_t segs, bool fine) {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return nst;
-  const int64_t units = n_items * Hkv, round = kWgPerCu * int64_t(cus);
+static int64_t choose_super_tiles(int64_t nst, int64_t n_items, int64_t Hkv, int64_t rows, int bits, int64_t max_tq,
+                                  int64_t max_tr, int64_t segs, bool fine) {
+  const int64_t cus = device_cus();
+  if (cus <= 0) return nst;
+  const int64_t units = n_items * Hkv, round = kWgPerCu * cus;
   const auto splits = [&](int64_t n) { return decode_mfma_num_splits(bits, n, max_tq, max_tr); };
   // Twice the super-tiles when that fits the launch into one round and `nst`
   // does not: a batch-1 32k context over 28 layers then runs as one full round
   // instead of ~1.9 (+3 % measured).
   if (units * splits(nst) > round) return units * splits(2 * nst) <= round ? 2 * nst : nst;
   if (!fine) return nst;
+  constexpr int64_t kTileCost[2][3] = {{15, 20, 30}, {14, 18, 26}};  // 2 and 4 bits, by workgroups on a CU
   const int64_t n_super = ceil_div(max_tq, decode_mfma_split_tokens(bits, 1));
+  const int64_t dense_cost = n_items / segs * Hkv * max_tr / 640;
+  const int64_t one_round = kCombineRound * combine_max_parts(rows);
   int64_t best = nst, best_cost = INT64_MAX;
   for (int64_t n = nst; n >= 1; --n) {
     const int64_t sp = ceil_div(n_super, n), groups = units * splits(n);
     if (sp == 0 || groups > min(round, kWgPerCu * kCus)) break;  // kCus: what the workspace is sized for
-    const int64_t tile = groups <= cus ? 15 : groups <= 2 * cus ? 20 : 30;
-    const int64_t cost = ceil_div(n_super, sp) * tile + segs * splits(n);
+    const int64_t tile = kTileCost[bits == 2 ? 0 : 1][groups <= cus ? 0 : groups <= 2 * cus ? 1 : 2];
+    const int64_t nflat = segs * splits(n);
+    const int64_t cost = max(ceil_div(n_super, sp) * tile, dense_cost) + nflat + max(nflat - one_round, int64_t(0));
     if (cost < best_cost) best = n, best_cost = cost;
   }
   return best;
@@ -1241,8 +1271,10 @@ int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single
                        int group_size, int64_t Hq, int64_t Hkv, int64_t Lq, int q_dtype, int res_dtype,
                        int out_dtype, float sm_scale, int64_t max_tq, int64_t max_tr, int64_t nst, int64_t segs,
                        bool fine, void *workspace, int64_t workspace_bytes, hipStream_t stream) {
+  UC_REQUIRE(segs >= 1 && n_items % segs == 0, "decode: %lld items do not form groups of %lld segments",
+             (long long)n_items, (long long)segs);
   const int64_t usual = nst;
-  nst = choose_super_tiles(nst, n_items, Hkv, bits, max_tq, max_tr, segs, fine);
+  nst = choose_super_tiles(nst, n_items, Hkv, Hq / Hkv * Lq, bits, max_tq, max_tr, segs, fine);
   const int64_t s_tok = decode_mfma_split_tokens(bits, nst);
   MfmaParams p{};
   p.Hq = Hq; p.Hkv = Hkv; p.Lq = Lq; p.group = Hq / Hkv; p.rows = p.group * Lq;
@@ -1295,14 +1327,14 @@ int launch_decode_mfma(const uc_kivi_item *items_dev, const uc_kivi_item *single
   }
   int rc = check_launch("decode (MFMA)");
   if (rc != UC_OK) return rc;
-  UC_REQUIRE(segs >= 1 && n_items % segs == 0, "decode: %lld items do not form groups of %lld segments",
-             (long long)n_items, (long long)segs);
-  // one block per (query group, KV head): enough parts that each takes its run
-  // of splits in less than one round of loads, as far as the block's threads go
-  // (a run of two rounds cost the 33 splits of a 32k segment 0.7 us of 17.9)
-  const int64_t nflat = segs * p.splits_total, span = ceil_div(p.rows * 16, int64_t(kWave)) * kWave;
+  // one block per (query group, KV head).  A split more in a part's run costs
+  // 0.17 us, a part more in the serial merge 0.6: runs of 12 splits for up to 4
+  // parts (one 2048-token segment at 4 bits, 16 splits: 10.2 us in 1 part, 9.5 in
+  // 2), of 16, the round of loads, beyond (one of 32768, 44 splits: 17.0 us in 8
+  // parts, 16.0 in 4)
+  const int64_t nflat = segs * p.splits_total, span = combine_span(p.rows), most = combine_max_parts(p.rows);
   int parts = 1;
-  while (nflat > kCombineRun * parts && 2 * parts * span <= kCombineMaxThreads) parts *= 2;
+  while (nflat > (parts < 4 ? 12 : kCombineRound) * parts && parts < most) parts *= 2;
   const auto combine = [&](auto f32_tag) {
     constexpr bool F32 = decltype(f32_tag)::value;
     const dim3 cgrid(static_cast<unsigned>(n_items / segs), static_cast<unsigned>(Hkv), F32 ? 2 : 1);

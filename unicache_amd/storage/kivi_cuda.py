@@ -95,7 +95,7 @@ def _decode_summary(cache: "PackedKIVICache", query: torch.Tensor, *, include_re
 
     device = nat.require_device(query, cache.key_code, what="Packed KIVI attention")
     q = query.contiguous()
-    lq, hq, d = map(int, q.shape)
+    lq, hq, d = q.shape
     tr = cache.residual_tokens if include_residual else 0
     out = torch.empty((lq, hq, d), dtype=out_dtype, device=device)
     lse = torch.empty((hq, lq), dtype=torch.float32, device=device)

@@ -362,7 +362,8 @@ int64_t uc_kivi_mq_workspace_bytes(int64_t heads_kv, int64_t head_dim, int64_t q
                                    int64_t residual_tokens);
 
 /*
- * uc_kivi_attn_mq over n_items (1..8) independent segments in one launch:
+ * uc_kivi_attn_mq over n_items (1..8) independent segments in one launch (or
+ * two, as uc_kivi_attn_mq_table):
  * item i attends its query_lens[i] queries (item.query / item.out /
  * item.lse, laid out as in uc_kivi_attn_mq) to its own packed prefix and
  * residual.  Every item shares bits, group_size, heads, head_dim and dtypes.
@@ -427,13 +428,13 @@ typedef struct uc_mq_query {
 } uc_mq_query;
 
 /*
- * uc_kivi_attn_mq_segments for up to 8 queries in one launch: query i attends,
- * as one softmax, the packed prefixes and residuals of items
- * packed_host[packed_begin .. + n_packed) and the dense segments
- * dense_host[dense_begin .. + n_dense) (runs of different queries may name the
- * same tensors).  Limits per call: 8 packed items and 16 dense segments,
- * counting each item's residual as one.  Results equal one
- * uc_kivi_attn_mq_segments call per query bit for bit.
+ * uc_kivi_attn_mq_segments for up to 8 queries in one launch (two where their
+ * lengths ask for both kinds of workgroup): query i attends, as one softmax,
+ * the packed prefixes and residuals of items packed_host[packed_begin .. +
+ * n_packed) and the dense segments dense_host[dense_begin .. + n_dense) (runs
+ * of different queries may name the same tensors).  Limits per call: 8 packed
+ * items and 16 dense segments, counting each item's residual as one.  Results
+ * equal one uc_kivi_attn_mq_segments call per query bit for bit.
  * Replaces: the per-sample loop of apply_static_physical_attention_batch
  * (adapters/bagel.py:773-980) for samples with long queries, whatever their
  * physical layout (CFG branches, H2O segments, several packed prefixes).

@@ -493,22 +493,60 @@ def test_mq_workgroups_of_one_and_two_halves(device, lq, tokens, dense, qdtype):
     assert_close(f32(part), f32(out)[5:700], max_abs=0.0313, mean_abs=5e-4, what="part of the rows")
 
 
-def test_mq_table_of_both_kinds(device):
-    # one table call whose queries take workgroups of one half and of two (two
-    # launches): each equals its own call bit for bit
-    from unicache_amd.storage.kivi_cuda import packed_segments_summary, packed_table_summaries
+def _kernels_of(run):
+    """Kernel launches of run(), counted as the nodes of its captured graph."""
 
+    import ctypes
+
+    with open("/proc/self/maps") as maps:  # the HIP runtime that torch loaded
+        hip = ctypes.CDLL(next(line.split()[-1] for line in maps if "libamdhip64" in line))
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        run()
+    count = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value
+
+
+# work items (128 rows x KV head) at 28/4 heads: 1200 queries 264, 1171 260 (an odd number of row blocks: the last
+# pair has one), 4098 900 (one half each); 90, 300, 500 and 1088 at most 240, 2345 516 (two halves each)
+@pytest.mark.parametrize("lens,odt,launches", [((300, 1200, 90), torch.bfloat16, 1), ((1171, 500), torch.float32, 1),
+                                               ((2345, 1171), torch.float16, 1), ((300, 4098), torch.bfloat16, 1),
+                                               ((1088, 1200), torch.float32, 2), ((1171, 1200), torch.float32, 1)])
+def test_mq_table_of_both_kinds(device, lens, odt, launches):
+    # one table call whose queries take workgroups of one half and of two: each
+    # query equals its own call bit for bit
     cache, _ = _pair(600, 100, 2, 32, 40, device)
-    entries, want = [], []
-    for i, lq in enumerate((300, 1200, 90)):
-        q = queries(lq, seed=101 + i).to(device)
-        dense = [tuple(x.to(device) for x in kv_pair(70 + i, seed=110 + i))]
-        out, lse = torch.empty_like(q), torch.empty((28, lq), dtype=torch.float32, device=device)
-        entries.append((q, out, lse, [cache], dense))
-        want.append(packed_segments_summary([cache], q, dense, dense_dtype=torch.bfloat16))
-    packed_table_summaries(entries, dense_dtype=torch.bfloat16)
-    for (_, out, lse, _, _), (o, x) in zip(entries, want):
-        assert torch.equal(out, o) and torch.equal(lse, x)
+    qs = [queries(lq, seed=101 + i).to(device) for i, lq in enumerate(lens)]
+    dense = [tuple(x.to(device) for x in kv_pair(70 + 64 * i, seed=110 + i)) for i in range(len(lens))]
+    codes = (nat.UC_BF16, nat.UC_BF16, nat.dtype_code(odt), 1.0 / math.sqrt(128))
+
+    def table(which, outs, lses):
+        queries_ = (nat.MqQuery * len(which))()
+        items, segs = (nat.KiviItem * len(which))(), (nat.DenseSegment * len(which))()
+        for j, i in enumerate(which):
+            queries_[j] = nat.MqQuery(qs[i].data_ptr(), outs[i].data_ptr(), lses[i].data_ptr(), lens[i], j, 1, j, 1)
+            items[j] = cache.native_item(None, None, None, residual_key_ptr=cache.residual_key.data_ptr(),
+                                         residual_value_ptr=cache.residual_value.data_ptr(),
+                                         residual_tokens=cache.residual_tokens)
+            key, value = dense[i]
+            segs[j] = nat.DenseSegment(key.data_ptr(), value.data_ptr(), int(key.shape[0]), 4 * 128, 128)
+        nat.call("uc_kivi_attn_mq_table", queries_, len(which), items, len(which), segs, len(which), 2, 32, 28, 4, 128,
+                 *codes, nat.stream(device))
+
+    def results():
+        return ([torch.full(q.shape, float("nan"), dtype=odt, device=device) for q in qs],
+                [torch.full((28, lq), float("nan"), device=device) for lq in lens])
+
+    want, got = results(), results()
+    for i in range(len(lens)):
+        table([i], *want)
+    assert _kernels_of(lambda: table(range(len(lens)), *got)) == launches
+    for i in range(len(lens)):
+        assert torch.isfinite(want[0][i].float()).all()
+        assert torch.equal(got[0][i], want[0][i]) and torch.equal(got[1][i], want[1][i]), f"query {i}"
 
 
 def test_mq_fp16_inputs(device):

@@ -4,10 +4,10 @@
 // softmax over every segment of a query in one launch.
 //
 // mq_attention_kernel: one workgroup owns 128 query rows of one KV head, 32 per
-// wave.  In launches that fill the chip it has 4 waves (HALVES 1) and two
-// workgroups share a CU: their barriers are their own, so the one's matrix
-// phases drift into the other's softmax.  In smaller launches it has 8 waves
-// (HALVES 2): waves 0-3 take half of the 64-key tiles (half of the packed
+// wave.  For a query with more of them than the chip has CUs it has 4 waves
+// (HALVES 1) and two workgroups share a CU: their barriers are their own, so the
+// one's matrix phases drift into the other's softmax.  For a smaller query it has
+// 8 waves (HALVES 2): waves 0-3 take half of the 64-key tiles (half of the packed
 // tiles, then part of the dense ones), waves 4-7 the rest, and the two merge at
 // the end (one_half has the rule and what both measured).
 // A tile's keys and values reach double-buffered LDS slots as fp16 or 16-bit
@@ -158,7 +158,9 @@ struct MqQuery {
   int64_t Lq, rows;   // rows = group * Lq query rows per KV head
   FastDiv lq;         // row -> (query head of the group, query position)
   int row_blocks;     // 128-row blocks per KV head
-  int per_xcd;        // work items (row block x KV head) per XCD
+  int by_rows;        // 8 waves: each half takes a row block of its own and every tile
+  int items;          // work items per KV head: a row block, or by_rows a pair of them
+  int per_xcd;        // work items per XCD
   int slot0;          // the query's first launch slot on every XCD
   int p0, np, d0, nd;  // its packed segments [p0, p0 + np) and dense ones [d0, d0 + nd)
   int pt, dt;          // its packed and dense 64-key tiles
@@ -659,12 +661,13 @@ __device__ __forceinline__ void convert_queries(u32x4 (&qf)[2][4]) {
     for (int kb = 0; kb < 4; ++kb) qf[qb][kb] = convert8<FROM, TO>(qf[qb][kb]);
 }
 
-// Work item of query Q: 128 query rows (row block rb) of KV head h over every
+// Work item b of query Q and KV head h: 128 query rows (row block b) over every
 // segment of the query.  Of two halves each takes half of the packed tiles (fp16
 // operands) and then dense tiles (dtype RD) up to n0 = ceil(tiles / 2) for
-// the first half.
+// the first half; or, by_rows, each takes a row block (2 b and 2 b + 1) and every
+// tile, in the order and with the arithmetic of a workgroup of one half.
 template <int HALVES, int BITS, int QD, int RD, int OD>
-__device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQuery &Q, int64_t h, int64_t rb) {
+__device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQuery &Q, int64_t h, int64_t b) {
   typedef typename DtypeOf<OD>::T OutT;
   __shared__ __align__(16) MqShared<HALVES, OutT> sh;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -672,14 +675,17 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
   const int half = HALVES == 2 ? wave / kHalfWaves : 0, hw = wave % kHalfWaves;
   const int tid_h = tid - half * kHalfThreads;
   const int r = lane & 15, kap = lane >> 4;
-  const int64_t row0 = rb * kMqRows + hw * kRowsPerWave;
+  const bool by_rows = HALVES == 2 && Q.by_rows != 0;
+  const bool split = HALVES == 2 && !by_rows;  // the halves share the rows and split the tiles
+  const bool second = split && half == 1;
+  const int64_t row0 = (by_rows ? 2 * b + half : b) * kMqRows + hw * kRowsPerWave;
 
-  // the first half's tiles, and the packed and dense ones among them
-  const int n_tiles = Q.pt + Q.dt, n0 = (n_tiles + HALVES - 1) / HALVES;
-  const int q0 = (Q.pt + HALVES - 1) / HALVES, d0 = n0 - q0;
-  const int pb = half ? q0 : 0, db = half ? d0 : 0;
-  const int n_pre = half ? Q.pt - q0 : q0;
-  const int count = n_pre + (half ? Q.dt - d0 : d0);
+  // the first half's tiles (or each half's), and the packed and dense ones among them
+  const int n_tiles = Q.pt + Q.dt, n0 = split ? (n_tiles + 1) / 2 : n_tiles;
+  const int q0 = split ? (Q.pt + 1) / 2 : Q.pt, d0 = n0 - q0;
+  const int pb = second ? q0 : 0, db = second ? d0 : 0;
+  const int n_pre = second ? Q.pt - q0 : q0;
+  const int count = n_pre + (second ? Q.dt - d0 : d0);
   const uint32_t sh_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)&sh));
   const uint32_t half_base = sh_base + half * 2 * kSlotBytes;
   const FragLane fl = frag_lane(half_base);
@@ -766,9 +772,9 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
   u32x4 qf[2][4];
   {
     u32x4 *qs = reinterpret_cast<u32x4 *>(sh.slot[0][1]) + hw * 8 * kWave + lane;
-    if (half == 0) {
+    if (!second) {
       load_queries(qf, Q, tb, h, row0);
-      if constexpr (HALVES == 2) {
+      if (split) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) qs[j * kWave] = qf[j / 4][j % 4];
       }
@@ -778,7 +784,7 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
       store_values<BITS>(pr, tid_h, half_base, magic);
     }
     __syncthreads();
-    if (half == 1) {
+    if (second) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) qf[j / 4][j % 4] = qs[j * kWave];
     }
@@ -836,7 +842,7 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
   // merge: the second half hands (O^T, m, l) of its lanes to the wave with the
   // same rows in the first half
   float *mg = sh.ep.mg[HALVES == 2 ? hw : 0];
-  if (HALVES == 2 && half == 1) {
+  if (second) {
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
 #pragma unroll
@@ -848,12 +854,13 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
     }
   }
   if constexpr (HALVES == 2) __syncthreads();
-  OutT *ob = sh.ep.ob + hw * kRowsPerWave * kRowPad;
-  if (half == 0) {
+  // normalised rows of the wave into its staging rows, and the LSE
+  auto finish = [&](OutT *ob, auto merge_tag) {
+    constexpr bool MERGE = decltype(merge_tag)::value;
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      const float m2 = HALVES == 2 ? mg[(64 + qb) * kWave + lane] : kNegInf;
-      const float l2 = HALVES == 2 ? mg[(66 + qb) * kWave + lane] : 0.0f;
+      const float m2 = MERGE ? mg[(64 + qb) * kWave + lane] : kNegInf;
+      const float l2 = MERGE ? mg[(66 + qb) * kWave + lane] : 0.0f;
       const float M = fmaxf(st.m[qb], m2);
       const float M_ref = M == kNegInf ? 0.0f : M;
       const float a1 = fast_exp2(st.m[qb] - M_ref), a2 = fast_exp2(m2 - M_ref);
@@ -863,9 +870,8 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
       for (int cb = 0; cb < 8; ++cb)
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const float o = HALVES == 2
-                              ? st.o[qb][cb][v] * a1 + mg[((qb * 8 + cb) * 4 + v) * kWave + lane] * a2
-                              : st.o[qb][cb][v];
+          const float o = MERGE ? st.o[qb][cb][v] * a1 + mg[((qb * 8 + cb) * 4 + v) * kWave + lane] * a2
+                                : st.o[qb][cb][v];
           store_from_f32<OD>(ob, (16 * qb + r) * kRowPad + 16 * cb + 4 * kap + v, o * inv);
         }
       const int64_t row = row0 + 16 * qb + r;
@@ -874,29 +880,44 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
         Q.lse[h * Q.rows + row] = l > 0.0f ? (M + log2f(l)) * kLn2 : kNegInf;
       }
     }
-  }
-  __syncthreads();
-  {  // each half writes its share of the 32 rows
+  };
+  // N of the wave's rows, from its staging row `first` on, to the output
+  auto write_rows = [&](const OutT *ob, int first, auto n_tag) {
+    constexpr int N = decltype(n_tag)::value;
     constexpr int kChunk = 16 / sizeof(OutT);  // elements per 16-byte store
     constexpr int kPerRow = kD / kChunk;
-    constexpr int kShare = kRowsPerWave / HALVES;
-    const OutT *obw = sh.ep.ob + hw * kRowsPerWave * kRowPad;
 #pragma unroll
-    for (int q = 0; q < kShare * kPerRow / kWave; ++q) {
-      const int idx = q * kWave + lane, rr = half * kShare + idx / kPerRow, cc = (idx % kPerRow) * kChunk;
+    for (int q = 0; q < N * kPerRow / kWave; ++q) {
+      const int idx = q * kWave + lane, rr = first + idx / kPerRow, cc = (idx % kPerRow) * kChunk;
       const int64_t row = row0 + rr;
       if (row >= Q.rows) continue;
       const uint32_t gq = fast_div(static_cast<uint32_t>(row), Q.lq);
       const int64_t g = gq, i = row - int64_t(gq) * Q.Lq;
       *reinterpret_cast<uint4 *>(static_cast<OutT *>(Q.out) + (i * tb.Hq + h * tb.group + g) * kD + cc) =
-          *reinterpret_cast<const uint4 *>(&obw[rr * kRowPad + cc]);
+          *reinterpret_cast<const uint4 *>(&ob[rr * kRowPad + cc]);
     }
+  };
+  OutT *ob = sh.ep.ob + hw * kRowsPerWave * kRowPad;
+  using AllRows = std::integral_constant<int, kRowsPerWave>;
+  if constexpr (HALVES == 2) {
+    if (split) {  // each half writes 16 of the 32 rows
+      if (half == 0) finish(ob, std::true_type{});
+      __syncthreads();
+      write_rows(ob, half * (kRowsPerWave / 2), std::integral_constant<int, kRowsPerWave / 2>{});
+      return;
+    }
+    // half 1 stages its rows in the merge area, which no one uses here
+    static_assert(sizeof(sh.ep.mg) >= kMqRows * kRowPad * sizeof(OutT), "a half's rows fit the merge area");
+    if (half == 1) ob = reinterpret_cast<OutT *>(sh.ep.mg) + hw * kRowsPerWave * kRowPad;
   }
+  finish(ob, std::false_type{});
+  __syncthreads();
+  write_rows(ob, 0, AllRows{});
 }
 
 // Launch slot id runs on XCD x = id % 8 as that XCD's slot j = id / 8.  Each
 // query owns slots [slot0, slot0 + per_xcd) of every XCD, and XCD x serves its
-// work items x * per_xcd .. (row blocks of KV head h at h * row_blocks ..): a
+// work items x * per_xcd .. (those of KV head h at h * items ..): a
 // contiguous run, mostly of one KV head, whose keys and values its own L2
 // then holds, and one eighth of every query.  Queries come longest first.
 template <int HALVES, int BITS, int QD, int RD, int OD>
@@ -907,8 +928,8 @@ __global__ __launch_bounds__(HALVES *kHalfThreads) __attribute__((amdgpu_waves_p
   while (qi + 1 < tb.n_queries && j >= tb.q[qi + 1].slot0) ++qi;
   const MqQuery &Q = tb.q[qi];
   const int w = x * Q.per_xcd + (j - Q.slot0);
-  if (w >= Q.row_blocks * tb.Hkv) return;  // uniform: the whole workgroup leaves
-  mq_attention_body<HALVES, BITS, QD, RD, OD>(tb, Q, w / Q.row_blocks, w % Q.row_blocks);
+  if (w >= Q.items * tb.Hkv) return;  // uniform: the whole workgroup leaves
+  mq_attention_body<HALVES, BITS, QD, RD, OD>(tb, Q, w / Q.items, w % Q.items);
 }
 
 }  // namespace
@@ -1072,21 +1093,21 @@ struct TableBuilder {
     const int64_t row_blocks = ceil_div(q.rows, int64_t(kMqRows));
     UC_REQUIRE(row_blocks * heads_kv < kOffsetLimit, "attn_mq: launch too large");
     q.row_blocks = static_cast<int>(row_blocks);
-    q.per_xcd = static_cast<int>(ceil_div(row_blocks * heads_kv, int64_t(kXcds)));
     return UC_OK;
   }
 
-  // Whether workgroups of one half (4 waves, every tile, two a CU) finish query
-  // `q` sooner than workgroups of two (8 waves, half the tiles each, one a CU).
-  // The choice looks at the query alone, so a query's result does not depend on
-  // the others of its launch.  Up to one work item per CU the one half would
-  // leave half of the chip's wave slots empty (GQA 28/4, two halves -> one: 240
-  // items over 2304 keys 49.0 -> 59.7 us); beyond, it wins (264 items over 2048
-  // keys 86.6 -> 73.9 us, 504 over 8192 290 -> 273 us, 900 over 8192 576 -> 528
-  // us), except where its second round of two items a CU is at most half full:
-  // 548 items over 8192 keys 430.7 -> 434.7 us, 768 434.6 -> 440.7 us.
+  // Whether query `q` takes workgroups of one half (4 waves, every tile, two a
+  // CU) rather than of two (8 waves, half the tiles each, one a CU).  The choice
+  // looks at the query alone, so a query's result does not depend on the others
+  // of its table.  Up to one work item per CU the one half would leave half of
+  // the chip's wave slots empty (GQA 28/4, two halves -> one: 240 items over 2304
+  // keys 49.0 -> 59.7 us); beyond, it wins (264 items over 2304 keys 92.6 -> 80.1
+  // us, over 9254 334 -> 303; 900 items 185.6 -> 159.7 and 668 -> 607), except
+  // where its second round of two items a CU is at most half full and the keys
+  // are many (516 items over 2304 keys 139.4 -> 130.1 us, but over 9254 502 ->
+  // 504, at 4 bits 504 -> 509).
+  static constexpr int64_t kCus = 256;  // of an MI355X
   bool one_half(const MqQuery &q) const {
-    constexpr int64_t kCus = 256;  // of an MI355X
     const int64_t items = q.row_blocks * heads_kv;
     return items > kCus && !(items > 2 * kCus && items <= 3 * kCus);
   }
@@ -1100,12 +1121,56 @@ struct TableBuilder {
     return n > 0;
   }
 
-  // Orders the queries longest first (segments stay where they are), assigns
-  // the launch slots and returns the grid size.
-  int64_t finish(float sm_scale) {
-    const auto work = [](const MqQuery &q) { return int64_t(q.pt + q.dt) * q.rows; };
+  // Whether a table of both kinds is one launch of 8-wave workgroups, in which
+  // the queries of one half give each half a row block (by_rows: the same bits),
+  // or two launches, in which they keep their separate barriers.  Estimates in
+  // rounds of the chip by two-half workgroups of the longest query: a by_rows
+  // workgroup takes 1.9 of them, a round of one-half workgroups 1.72 (0.64 of
+  // that when half of it or less is full); the one launch packs its workgroups to
+  // about 92 % and ends on whole rounds.  In one launch and in two, 28/4 heads
+  // over 2304 keys: 1200 queries with 300 more 87.7 and 128.4 us, with 2400 179
+  // and 221, with 1088 133.0 and 129.8; 4098 with 300 182 and 208, with 1088 219
+  // and 210.
+  bool together() const {
+    int64_t longest = 0, ones = 0, twos = 0;          // tiles; one-half and two-half workgroups
+    double pair_work = 0, one_work = 0, two_work = 0;  // by_rows, one-half and two-half ones weighted by their tiles
+    for (int i = 0; i < t.n_queries; ++i) longest = max(longest, int64_t(t.q[i].pt + t.q[i].dt));
+    for (int i = 0; i < t.n_queries; ++i) {
+      const MqQuery &q = t.q[i];
+      const double w = double(q.pt + q.dt) / longest;
+      const int64_t n = q.row_blocks * heads_kv;
+      if (one_half(q)) {
+        ones += n;
+        one_work += w * n;
+        pair_work += w * ((q.row_blocks + 1) / 2) * heads_kv;
+      } else {
+        twos += n;
+        two_work += w * n;
+      }
+    }
+    if (ones == 0 || twos == 0) return false;
+    const int64_t rest = ones % (2 * kCus);
+    const double rounds = ones / (2 * kCus) + (rest == 0 ? 0.0 : rest <= kCus ? 0.64 : 1.0);
+    const double apart = 1.72 * rounds * one_work / ones + ceil_div(twos, kCus) * two_work / twos;
+    return ceil((1.9 * pair_work + two_work) / (0.92 * kCus)) < apart;
+  }
+
+  // Orders the queries longest first (segments stay where they are; by_rows
+  // workgroups, which take every tile, before those that take half of them),
+  // assigns the launch slots and returns the grid size.
+  int64_t finish(float sm_scale, bool one) {
+    for (int i = 0; i < t.n_queries; ++i) {
+      MqQuery &q = t.q[i];
+      q.by_rows = !one && one_half(q);
+      q.items = q.by_rows ? (q.row_blocks + 1) / 2 : q.row_blocks;
+      q.per_xcd = static_cast<int>(ceil_div(int64_t(q.items) * heads_kv, int64_t(kXcds)));
+    }
+    const auto before = [](const MqQuery &a, const MqQuery &b) {
+      if (a.by_rows != b.by_rows) return a.by_rows > b.by_rows;
+      return int64_t(a.pt + a.dt) * a.rows > int64_t(b.pt + b.dt) * b.rows;
+    };
     for (int i = 1; i < t.n_queries; ++i)
-      for (int j = i; j > 0 && work(t.q[j]) > work(t.q[j - 1]); --j) std::swap(t.q[j], t.q[j - 1]);
+      for (int j = i; j > 0 && before(t.q[j], t.q[j - 1]); --j) std::swap(t.q[j], t.q[j - 1]);
     int slots = 0;
     for (int i = 0; i < t.n_queries; ++i) {
       t.q[i].slot0 = slots;
@@ -1122,10 +1187,11 @@ struct TableBuilder {
 
 int mq_launch(const TableBuilder &all, int bits, int q_dtype, int res_dtype, int out_dtype, float sm_scale,
               hipStream_t stream, const char *what) {
-  for (const bool one : {true, false}) {  // one launch, or two where the queries' kinds of workgroup differ
+  const bool together = all.together();
+  for (const bool one : {true, false}) {  // at most one launch of each kind of workgroup
     TableBuilder b = all;
-    if (!b.keep(one)) continue;
-    const int64_t grid = b.finish(sm_scale);
+    if (together ? one : !b.keep(one)) continue;
+    const int64_t grid = b.finish(sm_scale, one);
     UC_REQUIRE(grid < kOffsetLimit, "%s: launch too large", what);
     attn_config(bits, q_dtype, res_dtype, out_dtype, [&](auto bb, auto qd, auto rd, auto od) {
       constexpr int B = decltype(bb)::value, Q = decltype(qd)::value, R = decltype(rd)::value, O = decltype(od)::value;

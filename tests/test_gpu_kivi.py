@@ -462,9 +462,9 @@ def test_non_finite_inputs_match_oracle(device, native):
     assert np.array_equal(f32(kivi_fake_quant_value(value.to(device), bits=2, group_size=32)), fv, equal_nan=True)
 
 
-# The dense rows after the packed ones: in the packed rows' launch (16-byte
-# units), in one of their own (unaligned rows; 8 bits; other layouts), by a copy
-# (rows that are not compact or not of the wanted type).
+# The dense rows after the packed ones: in the packed rows' launch, in one of
+# their own (8 bits; fp32; other layouts), by a copy (rows that are not compact or
+# not of the wanted type).
 @pytest.mark.parametrize("bits,dtype", [(2, torch.bfloat16), (4, torch.float16), (4, torch.float32), (8, torch.bfloat16)])
 @pytest.mark.parametrize("rows,form", [(1, "compact"), (33, "compact"), (129, "shifted"), (40, "strided"), (7, "float32")])
 def test_dequantize_residual_rows(device, bits, dtype, rows, form):
@@ -488,3 +488,32 @@ def test_dequantize_residual_rows(device, bits, dtype, rows, form):
         rk, rv = torch.empty_like(got[0][:192]), torch.empty_like(got[1][:192])
         cache.dequantize_into(rk, rv, start=0, stop=192, output_offset=0)
         assert torch.equal(got[0][:192], rk) and torch.equal(got[1][:192], rv)
+
+
+@pytest.mark.parametrize("dtype,head_dim,rows", [(torch.bfloat16, 20, 5), (torch.float32, 20, 5), (torch.float16, 8, 1),
+                                                 (torch.bfloat16, 128, 300)])
+def test_restore_row_forms(device, dtype, head_dim, rows):
+    # the dense rows by themselves: 16-byte units where a row's channels are
+    # contiguous and a multiple of 16 bytes, else elements (20 16-bit channels;
+    # channels that are not contiguous), into rows of any alignment and stride
+    key, value = (x[..., :head_dim].contiguous() for x in kv_pair(16 + rows, heads=3, seed=70, dtype=dtype))
+    cache = PackedKIVICache.from_dense(key.to(device), value.to(device), logical_token_ids=torch.arange(16 + rows),
+                                       token_type_id=0, k_bits=8, v_bits=8, group_size=4, residual_length=rows)
+    assert cache.quantized_tokens == 16 and cache.residual_tokens == rows
+    plain = [torch.empty(16, 3, head_dim, dtype=dtype, device=device) for _ in range(2)]
+    cache.dequantize_into(*plain, start=0, stop=16, output_offset=0)
+    n = (16 + rows) * 3 * head_dim
+    for form in ("compact", "shifted", "heads first", "channels first"):
+        outs = []
+        for _ in range(2):
+            buf = torch.full((n + 1,), 7.0, dtype=dtype, device=device)[1 if form == "shifted" else 0:][:n]
+            if form == "heads first":
+                outs.append(buf.view(3, 16 + rows, head_dim).transpose(0, 1))
+            elif form == "channels first":
+                outs.append(buf.view(head_dim, 3, 16 + rows).permute(2, 1, 0))
+            else:
+                outs.append(buf.view(16 + rows, 3, head_dim))
+        cache._restore("uc_kivi_restore", cache.key_code.device, *outs, 0, 16, 0, cache.residual_key.data_ptr(),
+                       cache.residual_value.data_ptr(), rows)
+        for out, src, packed in zip(outs, (key, value), plain):
+            assert torch.equal(out[16:].cpu(), src[16:]) and torch.equal(out[:16], packed), form

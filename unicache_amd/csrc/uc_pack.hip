@@ -733,9 +733,11 @@ struct DequantArgs {
   int64_t res_rows;
 };
 
-// The dense rows of a tensor into the output rows after the packed ones, one
-// unit of sizeof(T) bytes a thread; units = head_dim * element bytes / sizeof(T).
-template <typename T>
+// The dense rows of a tensor into the output rows after the packed ones, UNIT
+// bytes a thread; units = head_dim * elem_bytes / UNIT.  Rows need no more than
+// their elements' alignment: the copies say so, and the memory system takes
+// unaligned 16-byte accesses.
+template <int UNIT>
 __device__ __forceinline__ void copy_residual(const DequantArgs &a, int64_t per_tensor, uint32_t units, int elem_bytes,
                                               int64_t idx) {
   if (idx >= 2 * per_tensor) return;
@@ -743,15 +745,21 @@ __device__ __forceinline__ void copy_residual(const DequantArgs &a, int64_t per_
   const uint32_t i = static_cast<uint32_t>(value ? idx - per_tensor : idx);
   const uint32_t q = i / units, u = i - q * units, heads = static_cast<uint32_t>(a.heads);
   const uint32_t n = q / heads, h = q - n * heads;
-  const int64_t ch = int64_t(u) * (sizeof(T) / elem_bytes);
-  char *out = static_cast<char *>(value ? a.out_value : a.out_key);
-  *reinterpret_cast<T *>(out + ((a.offset + a.count + n) * a.o_st + h * a.o_sh + ch * a.o_sd) * elem_bytes) =
-      static_cast<const T *>(value ? a.res_value : a.res_key)[i];
+  const int64_t ch = int64_t(u) * (UNIT / elem_bytes);
+  char *out = static_cast<char *>(value ? a.out_value : a.out_key) +
+              ((a.offset + a.count + n) * a.o_st + h * a.o_sh + ch * a.o_sd) * elem_bytes;
+  const char *in = static_cast<const char *>(value ? a.res_value : a.res_key) + int64_t(i) * UNIT;
+  struct Bytes {
+    unsigned char b[UNIT];
+  } x;
+  __builtin_memcpy(&x, in, UNIT);
+  __builtin_memcpy(out, &x, UNIT);
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void copy_residual_kernel(DequantArgs a, int64_t per_tensor) {
-  copy_residual<T>(a, per_tensor, static_cast<uint32_t>(a.head_dim), sizeof(T), int64_t(blockIdx.x) * 256 + threadIdx.x);
+template <int UNIT>
+__global__ __launch_bounds__(256) void copy_residual_kernel(DequantArgs a, int64_t per_tensor, uint32_t units,
+                                                            int elem_bytes) {
+  copy_residual<UNIT>(a, per_tensor, units, elem_bytes, int64_t(blockIdx.x) * 256 + threadIdx.x);
 }
 
 // One thread per output element (token, head, channel); keys and values are
@@ -987,7 +995,7 @@ __global__ __launch_bounds__(256) void dequant_kv_kernel(DequantArgs a, int64_t 
   else if (b < key_blocks + value_blocks)
     dequant_value_native_block<BITS, OD, VEC>(a, b - key_blocks);
   else
-    copy_residual<uint4>(a, a.res_rows * a.heads * a.head_dim / 8, static_cast<uint32_t>(a.head_dim / 8), 2,
+    copy_residual<16>(a, a.res_rows * a.heads * a.head_dim / 8, static_cast<uint32_t>(a.head_dim / 8), 2,
                          (b - key_blocks - value_blocks) * 256 + threadIdx.x);
 }
 
@@ -1365,22 +1373,28 @@ int dequant(const void *key_code, int64_t kc_sh, int64_t kc_sd, int64_t kc_sw,
   a.sd = stats_dtype; a.od = out_dtype;
   a.res_key = res_key; a.res_value = res_value; a.res_rows = res_rows;
   hipStream_t s = as_stream(stream);
-  // the dense rows by themselves, where no launch below takes them along
+  const int out_bytes = out_dtype == UC_FP32 ? 4 : 2;
+  // the dense rows by themselves, where no launch below takes them along: 16
+  // bytes a thread wherever a row's channels are contiguous and fill them (20000
+  // fp32 rows after 4096 packed tokens: an element a thread 52.0 us, two device
+  // copies 40.1, 16 bytes a thread 39.4)
   auto residual = [&] {
     if (res_rows == 0) return;
-    const int64_t per_tensor = res_rows * heads * head_dim;
+    const int unit = o_sd == 1 && head_dim * out_bytes % 16 == 0 ? 16 : out_bytes;
+    const int64_t units = head_dim * out_bytes / unit, per_tensor = res_rows * heads * units;
     const dim3 grid(static_cast<unsigned>(ceil_div(2 * per_tensor, int64_t(256))));
-    if (out_dtype == UC_FP32)
-      hipLaunchKernelGGL((copy_residual_kernel<uint32_t>), grid, dim3(256), 0, s, a, per_tensor);
-    else
-      hipLaunchKernelGGL((copy_residual_kernel<uint16_t>), grid, dim3(256), 0, s, a, per_tensor);
+    const auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a, per_tensor, static_cast<uint32_t>(units), out_bytes);
+    };
+    if (unit == 16) go(copy_residual_kernel<16>);
+    else if (unit == 4) go(copy_residual_kernel<4>);
+    else go(copy_residual_kernel<2>);
   };
   if (count == 0) {
     residual();
     return check_launch(entry);
   }
   // native 2/4-bit layout with pairwise-aligned unit-stride output rows
-  const int out_bytes = out_dtype == UC_FP32 ? 4 : 2;
   const bool out_ok = o_sd == 1 && o_st % 2 == 0 && o_sh % 2 == 0 && head_dim % 32 == 0 &&
                       (out_key == nullptr || aligned(out_key, 2 * out_bytes)) &&
                       (out_value == nullptr || aligned(out_value, 2 * out_bytes));
@@ -1410,10 +1424,9 @@ int dequant(const void *key_code, int64_t kc_sh, int64_t kc_sd, int64_t kc_sw,
         const int64_t runs = ceil_div(words, int64_t(kDqOctetWords));
         const int64_t key_blocks = ceil_div(heads * runs * (head_dim / 8), int64_t(256));
         const int64_t value_blocks = ceil_div(heads * count * (head_dim * v_bits / 32), int64_t(256));
-        // the dense rows as well, where they move in 16-byte units: a cache of
-        // 20353 tokens and 32 dense rows was three launches and 18.0 us
-        const bool along = res_rows > 0 && aligned(res_key, 16) && aligned(res_value, 16);
-        const int64_t res_blocks = along ? ceil_div(2 * (res_rows * heads * head_dim / 8), int64_t(256)) : 0;
+        // the dense rows as well, in 16-byte units: a cache of 20353 tokens and 32
+        // dense rows was three launches and 18.0 us
+        const int64_t res_blocks = ceil_div(2 * (res_rows * heads * head_dim / 8), int64_t(256));
         const dim3 grid(static_cast<unsigned>(key_blocks + value_blocks + res_blocks));
         auto go_kv = [&](auto sd_tag) {
           constexpr int SD = decltype(sd_tag)::value;
@@ -1426,7 +1439,6 @@ int dequant(const void *key_code, int64_t kc_sh, int64_t kc_sd, int64_t kc_sw,
         };
         if (stats_dtype == UC_BF16) go_kv(std::integral_constant<int, UC_BF16>{});
         else go_kv(std::integral_constant<int, UC_FP16>{});
-        if (!along) residual();
         return;
       }
       if (octet) {

@@ -517,3 +517,29 @@ def test_restore_row_forms(device, dtype, head_dim, rows):
                        cache.residual_value.data_ptr(), rows)
         for out, src, packed in zip(outs, (key, value), plain):
             assert torch.equal(out[16:].cpu(), src[16:]) and torch.equal(out[:16], packed), form
+
+
+def test_dequantize_keeps_what_residual_rows_carry(device):
+    # a lazily negated view has other values than its memory; tangents and
+    # gradients of the residual rows reach the restored ones
+    from torch.autograd import forward_ad
+
+    key, value = kv_pair(192 + 5, seed=80)
+    cache = PackedKIVICache.from_dense(key.to(device), value.to(device), logical_token_ids=torch.arange(197),
+                                       token_type_id=0, k_bits=4, v_bits=4, group_size=64, residual_length=5,
+                                       backend="cuda")
+    rows = cache.residual_key
+    cache.residual_key = torch._neg_view(rows)
+    assert torch.equal(cache.dequantize()[0][192:], -rows)
+    ones = torch.ones_like(rows)
+
+    def restored(x):
+        cache.residual_key = x
+        return cache.dequantize()[0]
+
+    with forward_ad.dual_level():
+        tangent = forward_ad.unpack_dual(restored(forward_ad.make_dual(rows, ones))).tangent
+        assert tangent is not None and torch.equal(tangent[192:], ones) and not tangent[:192].any()
+    tracked = rows.clone().requires_grad_()
+    restored(tracked)[192:].float().sum().backward()
+    assert torch.equal(tracked.grad, ones)

@@ -25,6 +25,7 @@ from dataclasses import dataclass
 from typing import Callable
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _native as nat
 
@@ -247,6 +248,13 @@ def _pack_native_at(ptrs, capacity: int, offset: int, key: torch.Tensor, value: 
     )
 
 
+def _is_plain(x: torch.Tensor) -> bool:
+    """Whether copying x by its address does what copy_ does, forward-mode
+    tangents aside: no subclass, no gradient, no lazily negated view."""
+
+    return type(x) is torch.Tensor and not x.requires_grad and not x.is_neg()
+
+
 def _native_block(capacity: int, heads: int, head_dim: int, k_bits: int, v_bits: int, group_size: int, device,
                   ids_dtype=None, ids_len: int = 0):
     """One allocation holding the token-major storage of `capacity` tokens and
@@ -411,7 +419,8 @@ class PackedKIVICache:
             return cls._from_dense_native(key, value, quantized, logical_token_ids, token_type_id, k_bits, v_bits,
                                           group_size)
         if quantized:
-            packed = _pack_reference_layout(key[:quantized], value[:quantized], k_bits=k_bits, v_bits=v_bits, group_size=group_size)
+            packed = _pack_reference_layout(key[:quantized], value[:quantized], k_bits=k_bits, v_bits=v_bits,
+                                            group_size=group_size)
             key_code, key_scale, key_minimum, value_code, value_scale, value_minimum = packed
         else:
             nat.require_device(key, value, what="KIVI physical cache")
@@ -708,10 +717,9 @@ class PackedKIVICache:
         key = torch.empty(shape, dtype=dtype, device=self.key_code.device)
         value = torch.empty_like(key)
         dense = self.residual_key, self.residual_value
-        if self.residual_tokens and all(
-            x.device == key.device and x.dtype == dtype and x.is_contiguous() and not x.requires_grad
-            and x.shape == (self.residual_tokens, *shape[1:]) and x.numel() <= 1 << 30
-            for x in dense
+        if self.residual_tokens and forward_ad._current_level < 0 and all(
+            _is_plain(x) and x.device == key.device and x.dtype == dtype and x.is_contiguous()
+            and x.shape == (self.residual_tokens, *shape[1:]) and x.numel() <= 1 << 30 for x in dense
         ):  # compact rows of the wanted type: the same launch copies them
             device = nat.require_device(self.key_code, key, what="KIVI dequantization")
             self._restore("uc_kivi_restore", device, key, value, 0, self.quantized_tokens, 0,

@@ -107,8 +107,12 @@ struct HsShared {
   float col[2][kHsWaves][kHsTile];
 };
 
-// s_waitcnt immediate (gfx9 layout): vmcnt <= n (6 bits), expcnt and lgkmcnt not waited on
-constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
+// s_waitcnt (gfx9 layout): vmcnt <= N, expcnt and lgkmcnt not waited on
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
 
 // The key rows [t_begin, t_end) of one KV head, streamed a tile at a time.
 // Rows past t_end fall outside the buffer resource and read as zero.
@@ -123,12 +127,14 @@ struct KeyStream {
     n_tiles = static_cast<int>((t_end - t_begin + kHsTile - 1) / kHsTile);
   }
 
-  // every thread: 4 loads of 16 B; wave w fills rows 16w .. 16w + 15 of the slot
+  // every thread: kLoads loads of 16 B; wave w fills rows 16w .. 16w + 15 of the slot
+  static constexpr int kLoads = kHsTile * 16 / kHsThreads;
+  static_assert(kLoads == 4 && kHsTile == 16 * kHsWaves, "the rows below");
   __device__ __forceinline__ void issue(HsShared &sh, int tile) const {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint4 *slot = sh.kt[tile % kHsStages];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < kLoads; ++j) {
       const int row = 16 * wave + 4 * j + (lane >> 4);
       const uint32_t off = static_cast<uint32_t>(tile * kHsTile + row) * row_bytes + 16u * ((lane & 15) ^ (row & 15));
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -143,47 +149,34 @@ struct KeyStream {
 
   // Tile i is in LDS for the whole workgroup; then the slot freed by tile i - 1
   // is refilled with tile i + kHsStages - 1.
-  __device__ __forceinline__ void acquire(HsShared &sh, int i) const {
-    const int ahead = min(n_tiles - 1, i + kHsStages - 2) - i;  // later tiles this thread still loads
-    static_assert(kHsStages <= 4, "vmcnt cases below");
-    if (ahead >= 2)
-      __builtin_amdgcn_s_waitcnt(kWaitVm8);
-    else if (ahead == 1)
-      __builtin_amdgcn_s_waitcnt(kWaitVm4);
-    else
-      __builtin_amdgcn_s_waitcnt(kWaitVm0);
-    __syncthreads();
-    if (i + kHsStages - 1 < n_tiles) issue(sh, i + kHsStages - 1);
-  }
-
-  // acquire() of a loop whose every tile before this one ended with exactly 16
-  // stores by this thread's wave.  Stores and loads share one in-order counter:
-  // a wait that counted the loads alone would also wait for the stores of the
-  // tiles before.  Issued after the loads of tile i: the stores of the last two
-  // tiles and the loads of tile i + 1.
-  __device__ __forceinline__ void acquire_past_stores(HsShared &sh, int i) const {
-    static_assert(kHsStages == 3, "the counts below");
-    const bool ahead = i + 1 < n_tiles;
-    if (i >= 2) {
-      if (ahead)
-        __builtin_amdgcn_s_waitcnt(wait_vm(4 + 32));
-      else
-        __builtin_amdgcn_s_waitcnt(wait_vm(32));
-    } else if (i == 1) {
-      if (ahead)
-        __builtin_amdgcn_s_waitcnt(wait_vm(4 + 16));
-      else
-        __builtin_amdgcn_s_waitcnt(wait_vm(16));
-    } else if (ahead) {
-      __builtin_amdgcn_s_waitcnt(wait_vm(4));
+  //
+  // STORES: with `stored` (uniform per wave) every tile before this one ended
+  // with that many stores by this thread's wave, and the wait leaves them in
+  // flight.  Stores and loads share one in-order counter, in which behind the
+  // loads of tile i stand the loads of the tiles after it and the stores of the
+  // last kHsStages - 1 tiles (fewer at the start).  More operations than counted
+  // make the wait longer, fewer would make it too short: the fences keep a tile's
+  // stores behind the loads issued before them.
+  template <int STORES = 0>
+  __device__ __forceinline__ void acquire(HsShared &sh, int i, bool stored = false) const {
+    static_assert(kHsStages == 3, "at most one later tile and the stores of two");
+    const bool ahead = i + 1 < n_tiles;  // this thread's loads of the next tile are issued
+    if (STORES > 0 && stored && i > 0) {
+      if (i >= 2) {
+        if (ahead) wait_vm<kLoads + 2 * STORES>();
+        else wait_vm<2 * STORES>();
+      } else {
+        if (ahead) wait_vm<kLoads + STORES>();
+        else wait_vm<STORES>();
+      }
     } else {
-      __builtin_amdgcn_s_waitcnt(wait_vm(0));
+      if (ahead) wait_vm<kLoads>();
+      else wait_vm<0>();
     }
     __syncthreads();
     if (i + kHsStages - 1 < n_tiles) issue(sh, i + kHsStages - 1);
+    if (STORES > 0) asm volatile("" ::: "memory");
   }
-
-  static constexpr int kWaitVm0 = wait_vm(0), kWaitVm4 = wait_vm(4), kWaitVm8 = wait_vm(8);
 };
 
 template <int DT>
@@ -403,7 +396,10 @@ __device__ __forceinline__ float from_lane_quads(float x, float from) {
 // 49.0 with whole lines, 47.4 with those waits (a fill of the size: 34).  Four
 // blocks a store (4 rows x 256 bytes) need 20 registers too many: 64 us.
 // Non-temporal stores: 81 us of half lines, 55 of whole ones.
-template <int DT>
+//
+// VEC: rows that start on 16 bytes and are a multiple of 4 keys long take 16-byte
+// stores throughout.  Other rows have a kernel without the whole-line form.
+template <int DT, bool VEC>
 __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3))) void qk_logits_kernel(HsParams p) {
   __shared__ __align__(16) HsShared sh;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -413,9 +409,6 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3)))
   const int64_t rb = it.rb, c = it.c, h = it.h;
   const int64_t t_begin = c * p.chunk, t_end = min(p.T, t_begin + p.chunk);
   const int64_t row0 = rb * kHsRows + wave * kHsRowsPerWave;
-  // 16-byte stores need rows that start on 16 bytes (uniform)
-  const bool vec = (p.T & 3) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0;
-
   // the first key tiles are requested before the query rows, so the two
   // latencies overlap
   const KeyStream ks(p, h, t_begin, t_end);
@@ -432,10 +425,10 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3)))
     const uint32_t i = static_cast<uint32_t>(row) - g * lq;
     ro[qb] = row < p.rows ? ((h * p.group + g) * p.Lq + i) * p.T : -1;
   }
-  // every row of the wave exists and rows take whole stores: full tiles end with
-  // exactly 16 stores, which acquire_past_stores counts on
-  // (a scalar: the branches on it hold the barrier)
-  const bool whole = __builtin_amdgcn_readfirstlane(vec && row0 + kHsRowsPerWave <= p.rows) != 0;
+  // every row of the wave exists: full tiles end with kTileStores stores.  They
+  // are of 16 bytes, so none can be merged.  (A scalar: uniform branches)
+  constexpr int kTileStores = VEC ? kHsTile / 16 * kHsQB : 0;
+  const bool whole = VEC && __builtin_amdgcn_readfirstlane(row0 + kHsRowsPerWave <= p.rows) != 0;
   // where this lane's first store of a block pair goes: row n & 7 of 16 qb,
   // keys 4k .. + 3 of the pair's first (n < 8) or second block; its other store
   // is 8 rows on (rows are contiguous: [Hq][Lq] of one KV head)
@@ -443,14 +436,11 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3)))
 #pragma unroll
   for (int qb = 0; qb < kHsQB; ++qb) pr[qb] = ro[qb] - (r & 8) * p.T + 4 * kap + 2 * (r & 8);
   for (int i = 0; i < ks.n_tiles; ++i) {
-    if (whole)
-      ks.acquire_past_stores(sh, i);
-    else
-      ks.acquire(sh, i);
+    ks.acquire<kTileStores>(sh, i, whole);
     const int64_t t0 = t_begin + int64_t(i) * kHsTile;
     const uint4 *kt = sh.kt[i % kHsStages];
-    if (whole && t0 + kHsTile <= t_end) {
-      for (int tb = 0; tb < 4; tb += 2) {
+    if (VEC && whole && t0 + kHsTile <= t_end) {
+      for (int tb = 0; tb < kHsTile / 16; tb += 2) {
         typename HsOp<DT>::V kf[2][4];
 #pragma unroll
         for (int u = 0; u < 2; ++u)
@@ -479,8 +469,10 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3)))
       }
       continue;
     }
-#pragma unroll
-    for (int tb = 0; tb < 4; ++tb) {
+    // (rolled to 2 beside the whole-line form: unrolled, the compiler splits the
+    // tile loop and 235 MB of logits take 41.9 us instead of 41.3)
+#pragma unroll VEC ? 2 : 4
+    for (int tb = 0; tb < kHsTile / 16; ++tb) {
       typename HsOp<DT>::V kf[4];
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) kf[kb] = key_frag<DT>(kt, 16 * tb + r, 4 * kb + kap);
@@ -492,8 +484,8 @@ __global__ __launch_bounds__(kHsThreads) __attribute__((amdgpu_waves_per_eu(3)))
         for (int kb = 0; kb < 4; ++kb) s = HsOp<DT>::mma(kf[kb], qf[qb][kb], s);
         if (ro[qb] < 0) continue;
         float *dst = p.logits + ro[qb] + t;
-        if (vec && t + 4 <= t_end) {
-          *reinterpret_cast<f4 *>(dst) = s * p.scale;
+        if (VEC) {  // chunks and T end on multiples of 4 keys
+          if (t < t_end) *reinterpret_cast<f4 *>(dst) = s * p.scale;
         } else {
 #pragma unroll
           for (int v = 0; v < 4; ++v)
@@ -619,13 +611,6 @@ __device__ __forceinline__ typename PvOp<VD>::V p_frag(const PRaw<PD> &raw, int6
       w[e] = uint32_t(PvOp<VD>::bits(x[2 * e])) | (uint32_t(PvOp<VD>::bits(x[2 * e + 1])) << 16);
   }
   return __builtin_bit_cast(typename PvOp<VD>::V, make_uint4(w[0], w[1], w[2], w[3]));
-}
-
-// s_waitcnt immediate (gfx9 layout): vmcnt <= n, expcnt and lgkmcnt not waited on
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
 template <int PD, int VD>
@@ -838,10 +823,11 @@ int launch_qk_logits_mfma(int dtype, const void *q, int64_t q_si, int64_t q_sh, 
   p.items = p.row_blocks * p.chunks * Hkv;
   p.per_xcd = ceil_div(p.items, int64_t(kXcds));
   const dim3 grid(static_cast<unsigned>(p.per_xcd * kXcds));
-  if (dtype == UC_FP16)
-    hipLaunchKernelGGL((qk_logits_kernel<UC_FP16>), grid, dim3(kHsThreads), 0, stream, p);
-  else
-    hipLaunchKernelGGL((qk_logits_kernel<UC_BF16>), grid, dim3(kHsThreads), 0, stream, p);
+  static_assert(kHsTile % 4 == 0, "chunks are whole tiles");
+  const bool vec = T % 4 == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0;
+  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kHsThreads), 0, stream, p); };
+  if (dtype == UC_FP16) go(vec ? qk_logits_kernel<UC_FP16, true> : qk_logits_kernel<UC_FP16, false>);
+  else go(vec ? qk_logits_kernel<UC_BF16, true> : qk_logits_kernel<UC_BF16, false>);
   return check_launch("uc_kivi_qk (MFMA logits)");
 }
 

@@ -8,7 +8,7 @@ from oracle import h2o as H
 from unicache_amd.core.decisions import PhysicalCacheRequest
 from unicache_amd.operators import KIVIPackedQuantizationOperator, H2OPhysicalGQAOperator
 from unicache_amd.storage import GQAH2OCache, PackedKIVICache
-from unicache_amd.storage import kivi_cuda
+from unicache_amd.storage import kivi_cuda, physical
 from unicache_amd.storage.tensor_backend import h2o_budget
 
 
@@ -30,6 +30,27 @@ def test_budget_matches_oracle(n):
     for params in ({"target_budget_ratio": 0.2, "recent_budget_fraction": 0.25},
                    {"target_budget_ratio": 0.5}, {"budget": 7, "recent_size": 3}, {"keep_k": 5}):
         assert h2o_budget(n, params) == H.budget(n, params)
+
+
+@pytest.mark.parametrize("capacity,heads,head_dim,k_bits,v_bits,group", [(96, 4, 128, 2, 2, 32), (128, 3, 64, 4, 2, 64),
+                                                                         (32, 1, 128, 2, 4, 16)])
+@pytest.mark.parametrize("ids", [None, (torch.int64, 77), (torch.int32, 5), (torch.uint8, 3)])
+def test_native_block_carves_the_native_storage(capacity, heads, head_dim, k_bits, v_bits, group, ids):
+    # the offsets _native_block computes by itself are those of the tensors of
+    # _native_specs carved one after the other, the ids slot after them
+    specs = physical._native_specs(capacity, heads, head_dim, k_bits, v_bits, group)
+    carved = physical._carve(specs + ([((ids[1],), ids[0])] if ids else []), "cpu")
+    want = physical._native_views(carved[:6], capacity, k_bits, group)
+    views, ptrs, slot = physical._native_block(capacity, heads, head_dim, k_bits, v_bits, group, "cpu", *(ids or ()))
+    for view, ptr, exp in zip(views, ptrs, want):
+        assert (view.shape, view.stride(), view.dtype) == (exp.shape, exp.stride(), exp.dtype)
+        assert view.data_ptr() == ptr and ptr - views[0].data_ptr() == exp.data_ptr() - want[0].data_ptr()
+    last = slot if ids else views[5]
+    if ids:
+        assert (slot.shape, slot.dtype) == ((ids[1],), ids[0])
+        assert slot.data_ptr() - views[0].data_ptr() == carved[6].data_ptr() - carved[0].data_ptr()
+    storage = views[0].untyped_storage()
+    assert last.data_ptr() + last.numel() * last.element_size() <= storage.data_ptr() + storage.nbytes()
 
 
 def test_cpu_tensors_fail_closed():

@@ -493,6 +493,30 @@ def test_mq_workgroups_of_one_and_two_halves(device, lq, tokens, dense, qdtype):
     assert_close(f32(part), f32(out)[5:700], max_abs=0.0313, mean_abs=5e-4, what="part of the rows")
 
 
+@pytest.mark.parametrize("dtype,tokens", [(torch.bfloat16, 4096), (torch.float16, 4096), (torch.bfloat16, 700)])
+def test_mq_one_half_is_as_close_as_two(device, dtype, tokens):
+    # 1200 queries (264 work items: one half) against two calls of 600 (132 items
+    # each: two halves) on the same rows: fp32 outputs no further from 64 bits
+    key, value = (x.to(device) for x in kv_pair(tokens, seed=190, dtype=dtype))
+    q = queries(1200, seed=191, dtype=dtype).to(device)
+
+    def attend(rows):
+        out = torch.empty(rows.shape, dtype=torch.float32, device=device)
+        seg = (nat.DenseSegment * 1)(nat.DenseSegment(key.data_ptr(), value.data_ptr(), tokens, 4 * 128, 128))
+        nat.call("uc_kivi_attn_mq_segments", (nat.KiviItem * 1)(), 0, seg, 1, rows.data_ptr(), out.data_ptr(), None, 2, 32,
+                 28, 4, 128, int(rows.shape[0]), nat.dtype_code(dtype), nat.dtype_code(dtype), nat.UC_FP32,
+                 1.0 / math.sqrt(128), nat.stream(device))
+        return out
+
+    one, two = attend(q), torch.cat([attend(q[:600]), attend(q[600:])])
+    assert not torch.equal(one, two)  # two kinds of workgroup
+    exact = torch.empty(1200, 28, 128, dtype=torch.float64, device=device)
+    for h in range(28):
+        k, v = key[:, h // 7].double().t().contiguous(), value[:, h // 7].double().contiguous()
+        exact[:, h] = torch.softmax((q[:, h].double().contiguous() @ k) / math.sqrt(128), -1) @ v
+    assert float((one - exact).norm()) <= float((two - exact).norm())
+
+
 def _kernels_of(run):
     """Kernel launches of run(), counted as the nodes of its captured graph."""
 

@@ -102,8 +102,14 @@ constexpr int kRowsPerWave = 32;
 constexpr int kMqRows = kHalfWaves * kRowsPerWave;  // query rows per workgroup
 // The reference of a query column is raised only when a logit exceeds it by
 // more than kSlack (log2 units): probabilities stay below 2^kSlack, and most
-// tiles need no rescale of the output accumulators.
-constexpr float kSlack = 8.0f;
+// tiles need no rescale of the output accumulators.  The key that sets the
+// reference weighs exactly 1; all others are rounded to the operand dtype.  Two
+// halves over the keys set two references, so a query of one half, with fewer
+// exact weights at the same slack, would be 1 to 3 % further from the 64-bit
+// result.  It raises its reference sooner instead: relative error of fp32 outputs
+// over 8192 bf16 keys 1.085e-3 in two halves, 1.123e-3 in one with a slack of 8,
+// 1.035e-3 with 5, for 0 to 1.4 % of the time (a slack of 4: 0.993e-3, up to 2.5 %).
+constexpr float kSlack = 8.0f, kSlackOne = 5.0f;
 
 // One 64-key tile in LDS: 64 rows of 256 B (16 chunks of 16 B) of keys and of
 // values.  Key row t keeps chunk c at position c ^ (t & 15): the 16 rows one
@@ -521,7 +527,7 @@ __device__ __forceinline__ u32x2 read_vt(uint32_t addr) {
 // of key half tp, so that it issues while the matrix cores are busy.
 template <int DT, int BUF, bool HOOK, class Hook>
 __device__ __forceinline__ void compute_tile(FragLane fl, const u32x4 (&qf)[2][4], int valid, float scale_log2,
-                                             MqState &st, Hook &&hook) {
+                                             float slack, MqState &st, Hook &&hook) {
   constexpr uint32_t kBuf = BUF * kSlotBytes;
   using Op = Mma<DT>;
   const int lane = threadIdx.x & 63;
@@ -568,7 +574,7 @@ __device__ __forceinline__ void compute_tile(FragLane fl, const u32x4 (&qf)[2][4
 #pragma unroll
       for (int v = 0; v < 4; ++v) mx = fmaxf(mx, acc[tb][qb][v]);
     mx = max_over_slices(mx) * scale_log2;  // the column's tile max, log2 units
-    if (__any(mx > st.m[qb] + kSlack)) {    // some column outgrew its reference: move it to the tile max
+    if (__any(mx > st.m[qb] + slack)) {    // some column outgrew its reference: move it to the tile max
       // (a wave-uniform branch; inside it every lane scales, by 1 where nothing moved)
       const float m_new = fmaxf(st.m[qb], mx);
       const float alpha = m_new == st.m[qb] ? 1.0f : fast_exp2(st.m[qb] - m_new);  // 0 while nothing is accumulated
@@ -678,6 +684,7 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
   const bool by_rows = HALVES == 2 && Q.by_rows != 0;
   const bool split = HALVES == 2 && !by_rows;  // the halves share the rows and split the tiles
   const bool second = split && half == 1;
+  const float slack = split ? kSlack : kSlackOne;
   const int64_t row0 = (by_rows ? 2 * b + half : b) * kMqRows + hw * kRowsPerWave;
 
   // the first half's tiles (or each half's), and the packed and dense ones among them
@@ -813,7 +820,7 @@ __device__ __forceinline__ void mq_attention_body(const MqTable &tb, const MqQue
     if (i < count) {
       // a packed tile's dequantization rides in the P.V MFMAs of the
       // previous (packed) tile
-      compute_tile<DT, BUF, NEXT_PACKED>(fl, qf, cur_valid, tb.scale_log2, st, hook);
+      compute_tile<DT, BUF, NEXT_PACKED>(fl, qf, cur_valid, tb.scale_log2, slack, st, hook);
     }
     cur_valid = next_valid;
   };

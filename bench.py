@@ -4,7 +4,7 @@ Workload: batched decode over 2-bit KIVI-packed KV,
 GQA 28/4, head_dim 128, 28 layers, batch 8, 8192 tokens per sequence (8064
 packed + 128 bf16 residual), one bf16 query token per sequence per step.
 A step is one decode pass over all 28 layers x 8 sequences: a single
-uc_kivi_attn_decode_batch launch (split-K partials + LSE combine) over 28
+uc_kivi_attn_decode_fine launch (split-K partials + LSE combine) over 28
 distinct layer buffers (755 MB, more than the 256 MB Infinity Cache).
 
 Prints one JSON line: metric value = algorithmic bytes moved per step / step
@@ -233,7 +233,7 @@ def time_steps_each(fn, steps, warmup, stream):
 def long_context_decode(device, steps, layers=LAYERS, tokens=32768):
     """Config 4's packed segment as a pure-packed variant: batch 1, 28 layers x
     32768 tokens (32640 packed 2-bit + 128 residual), one decode step = one
-    uc_kivi_attn_decode_batch over the 28 layers."""
+    uc_kivi_attn_decode_fine over the 28 layers."""
 
     from unicache_amd.storage import PackedKIVICache
     from unicache_amd.storage.decode import KiviDecodeBatch
@@ -396,7 +396,7 @@ def mixed_decode(device, steps, layers=LAYERS):
     20224 packed 2-bit + 128 fp16 residual) and the bf16 tokens kept dense (128
     protected + instruction 4096 -> 819 and ViT 8192 -> 1638 after H2O at a 20%
     budget) attended as one softmax; all 28 layers in one
-    uc_kivi_attn_decode_segments launch.
+    uc_kivi_attn_decode_fine launch.
 
     Two figures: the decode step itself (the static table, timed back to
     back), and the 64-step decode loop of the configuration: each step runs
@@ -481,7 +481,7 @@ def mixed_decode(device, steps, layers=LAYERS):
     return {
         "workload": f"config 4 decode step: {layers} layers x (VAE {vae} tokens: {packed0} packed "
                     f"2-bit + {window0} fp16 residual | {dense_tokens} dense tokens: 128 protected "
-                    "+ 819 + 1638 H2O-retained), batch 1, Lq=1, one uc_kivi_attn_decode_segments launch",
+                    "+ 819 + 1638 H2O-retained), batch 1, Lq=1, one uc_kivi_attn_decode_fine launch",
         "ms_per_step": round(ms, 5),
         "gbs": round(gbs, 1),
         "frac_of_hbm_peak": round(gbs / HBM_PEAK_GBS, 4),
@@ -916,7 +916,7 @@ def main():
             "unit": "GB/s",
             "frac": round(value / HBM_PEAK_GBS, 4),
             "traffic": MEASURED_TRAFFIC_BYTES if args.layers == LAYERS else None,
-            "kernel": "uc_kivi_attn_decode_batch = decode_mfma_kernel + decode_mfma_combine, one call per step",
+            "kernel": "uc_kivi_attn_decode_fine = decode_mfma_kernel + decode_mfma_combine, one call per step",
             "bytes_per_launch": step_bytes,
         },
         "per_layer_launches_gbs": round(step_bytes / (ms_layers * 1e-3) / 1e9, 2),

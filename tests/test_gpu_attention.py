@@ -244,6 +244,57 @@ def test_decode_results_do_not_depend_on_workspace(device, bits, group, tokens, 
         summary("uc_kivi_attn_decode_fine", 4)
 
 
+@pytest.mark.parametrize("bits,group,lengths", [(2, 32, (2500,) * 4), (4, 64, (4500,) * 4), (2, 32, (2048, 700, 4500, 287))])
+def test_decode_tables_equal_single_calls(device, bits, group, lengths):
+    # the C calls over device tables: a small batch gives segments as long as its
+    # longest the bits of their own calls, and a group of segments has those of
+    # uc_kivi_attn_decode_segments_host
+    import ctypes
+
+    caches, segs = zip(*(_pair(t, 200 + i, bits, group, 100, device) for i, t in enumerate(lengths)))
+    qs = [queries(1, seed=210 + i).to(device) for i in range(4)]
+    args = (bits, group, 28, 4, 128, 1, nat.UC_BF16, nat.UC_BF16, nat.UC_BF16, 1.0 / math.sqrt(128))
+    ws = nat.workspace(device, 8 << 20)
+    room = (ws.data_ptr(), 8 << 20, nat.stream(device))
+
+    def results():
+        return ([torch.full_like(q, float("nan")) for q in qs],
+                [torch.full((28, 1), float("nan"), device=device) for _ in qs])
+
+    def items(outs, lses, query=None):
+        table = (nat.KiviItem * 4)()
+        for i, c in enumerate(caches):
+            q = qs[i] if query is None else query
+            table[i] = c.native_item(q.data_ptr(), outs[i].data_ptr(), lses[i].data_ptr(),
+                                     residual_key_ptr=c.residual_key.data_ptr(),
+                                     residual_value_ptr=c.residual_value.data_ptr(),
+                                     residual_tokens=c.residual_tokens)
+        raw = bytearray(ctypes.string_at(ctypes.addressof(table), ctypes.sizeof(table)))
+        return table, torch.frombuffer(raw, dtype=torch.uint8).to(device)
+
+    tokens = (max(c.quantized_tokens for c in caches), max(c.residual_tokens for c in caches))
+    want, got = results(), results()
+    host, _ = items(*want)
+    for i in range(4):
+        nat.call("uc_kivi_attn_decode", host[i], *args, *room)
+        check_summary(want[0][i], want[1][i], segs[i], qs[i].cpu(), what=f"item {i}")
+    _, table = items(*got)
+    nat.call("uc_kivi_attn_decode_batch", table.data_ptr(), 4, *args, *tokens, *room)
+    for i in range(4):
+        check_summary(got[0][i], got[1][i], segs[i], qs[i].cpu(), what=f"batch item {i}")
+        if lengths[i] == lengths[0] == max(lengths):
+            assert torch.equal(got[0][i], want[0][i]) and torch.equal(got[1][i], want[1][i]), f"item {i}"
+    host, _ = items(*want, query=qs[0])
+    nat.call("uc_kivi_attn_decode_segments_host", host, 4, *args, *room)
+    _, table = items(*got, query=qs[0])
+    nat.call("uc_kivi_attn_decode_segments", table.data_ptr(), 4, 4, *args, *tokens, *room)
+    assert torch.equal(got[0][0], want[0][0]) and torch.equal(got[1][0], want[1][0])
+    pairs = [K.dequantize(seg, "fp32") for seg in segs]
+    eo, el = A.attention_summary(f32(qs[0]), np.concatenate([k for k, _ in pairs]), np.concatenate([v for _, v in pairs]))
+    assert_close(f32(got[0][0]), eo, what="out")
+    assert_close(f32(got[1][0]), el, max_abs=1e-2, mean_abs=1e-3, what="lse")
+
+
 @pytest.mark.parametrize("bits,group,hq,lq,lengths", [(2, 32, 28, 1, (2048,)), (2, 64, 28, 2, (2048, 1024, 256)),
                                                       (4, 64, 16, 1, (1024,)), (4, 128, 32, 2, (8192,) * 4),
                                                       (2, 32, 12, 1, (32768, 512)), (2, 32, 32, 1, (8192,) * 8)])

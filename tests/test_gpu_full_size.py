@@ -2,7 +2,7 @@
 shapes bench.py times), complementing the reduced-size parity tests:
 
 - config 1: the 224-item (28 layers x batch 8, 8192 tokens) decode table in
-  one uc_kivi_attn_decode_batch launch, sampled items against the oracle;
+  one uc_kivi_attn_decode_fine launch, sampled items against the oracle;
 - config 2: the whole editing pass, 1088 queries over 2304 keys, 2- and 4-bit;
 - config 3: H2O scores of 512 queries over 4096 keys, then the per-segment
   selection -- indices asserted bit-exact at a seed whose selection margin

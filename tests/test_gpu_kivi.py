@@ -543,3 +543,20 @@ def test_dequantize_keeps_what_residual_rows_carry(device):
     tracked = rows.clone().requires_grad_()
     restored(tracked)[192:].float().sum().backward()
     assert torch.equal(tracked.grad, ones)
+
+
+@pytest.mark.parametrize("bits,tokens", [(2, 32768), (4, 32700)])
+def test_pack_of_a_long_segment_matches_oracle(device, bits, tokens):
+    # every code word and statistic of a 32k segment, not only its start
+    key, value = kv_pair(tokens, seed=90 + bits)
+    cache = PackedKIVICache.from_dense(key.to(device), value.to(device), logical_token_ids=torch.arange(tokens),
+                                       token_type_id=3, k_bits=bits, v_bits=bits, group_size=32, residual_length=128,
+                                       backend="cuda")
+    seg = K.from_dense(f32(key), f32(value), k_bits=bits, v_bits=bits, group_size=32, residual_length=128, native=True)
+    for name in ("key_code", "value_code"):
+        assert np.array_equal(getattr(cache, name).cpu().numpy(), getattr(seg, name)), name
+    for name in ("key_scale", "key_minimum", "value_scale", "value_minimum"):
+        assert np.array_equal(f32(getattr(cache, name)), np.asarray(getattr(seg, name), dtype=np.float32)), name
+    n = cache.quantized_tokens
+    assert torch.equal(cache.residual_key.cpu(), key[n:]) and torch.equal(cache.residual_value.cpu(), value[n:])
+    assert torch.equal(cache.logical_token_ids.cpu(), torch.arange(tokens))

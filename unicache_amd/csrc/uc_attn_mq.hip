@@ -1108,8 +1108,8 @@ struct TableBuilder {
   // looks at the query alone, so a query's result does not depend on the others
   // of its table.  Up to one work item per CU the one half would leave half of
   // the chip's wave slots empty (GQA 28/4, two halves -> one: 240 items over 2304
-  // keys 49.0 -> 59.7 us); beyond, it wins (264 items over 2304 keys 92.6 -> 80.1
-  // us, over 9254 334 -> 303; 900 items 185.6 -> 159.7 and 668 -> 607), except
+  // keys 49.0 -> 59.7 us); beyond, it wins (264 items over 2304 keys 92.9 -> 81.2
+  // us, over 9254 335 -> 301; 900 items 187 -> 164 and 670 -> 620), except
   // where its second round of two items a CU is at most half full and the keys
   // are many (516 items over 2304 keys 139.4 -> 130.1 us, but over 9254 502 ->
   // 504, at 4 bits 504 -> 509).

@@ -248,13 +248,6 @@ def _pack_native_at(ptrs, capacity: int, offset: int, key: torch.Tensor, value: 
     )
 
 
-def _is_plain(x: torch.Tensor) -> bool:
-    """Whether copying x by its address does what copy_ does, forward-mode
-    tangents aside: no subclass, no gradient, no lazily negated view."""
-
-    return type(x) is torch.Tensor and not x.requires_grad and not x.is_neg()
-
-
 def _native_block(capacity: int, heads: int, head_dim: int, k_bits: int, v_bits: int, group_size: int, device,
                   ids_dtype=None, ids_len: int = 0):
     """One allocation holding the token-major storage of `capacity` tokens and
@@ -696,14 +689,14 @@ class PackedKIVICache:
         kcs, kss, vcs, vss = self._code_strides()
         nat.call(
             entry,
-            nat.ptr(self.key_code) if out_key is not None else None, *map(int, kcs),
-            self.key_scale.data_ptr(), self.key_minimum.data_ptr(), *map(int, kss),
-            nat.ptr(self.value_code) if out_value is not None else None, *map(int, vcs),
-            self.value_scale.data_ptr(), self.value_minimum.data_ptr(), *map(int, vss),
+            nat.ptr(self.key_code) if out_key is not None else None, *kcs,
+            self.key_scale.data_ptr(), self.key_minimum.data_ptr(), *kss,
+            nat.ptr(self.value_code) if out_value is not None else None, *vcs,
+            self.value_scale.data_ptr(), self.value_minimum.data_ptr(), *vss,
             nat.dtype_code(self.key_scale.dtype), self.num_kv_heads, self.head_dim,
             self.k_bits, self.v_bits, self.group_size, int(start), int(stop),
             nat.ptr(out_key), nat.ptr(out_value), nat.dtype_code(ref.dtype),
-            *map(int, ref.stride()), int(output_offset), *residual, nat.stream(device),
+            *ref.stride(), int(output_offset), *residual, nat.stream(device),
         )
 
     def dequantize(self, dtype: torch.dtype | None = None) -> tuple[torch.Tensor, torch.Tensor]:
@@ -717,10 +710,14 @@ class PackedKIVICache:
         key = torch.empty(shape, dtype=dtype, device=self.key_code.device)
         value = torch.empty_like(key)
         dense = self.residual_key, self.residual_value
+        # compact rows of the wanted type: the same launch copies them, by address
+        # (subclasses, tracked rows, lazily negated views and forward-mode tangents
+        # carry more than their memory and are copied by copy_)
         if self.residual_tokens and forward_ad._current_level < 0 and all(
-            _is_plain(x) and x.device == key.device and x.dtype == dtype and x.is_contiguous()
-            and x.shape == (self.residual_tokens, *shape[1:]) and x.numel() <= 1 << 30 for x in dense
-        ):  # compact rows of the wanted type: the same launch copies them
+            type(x) is torch.Tensor and x.device == key.device and x.dtype == dtype and x.is_contiguous()
+            and not x.requires_grad and not x.is_neg() and x.shape == (self.residual_tokens, *shape[1:])
+            and x.numel() <= 1 << 30 for x in dense
+        ):
             device = nat.require_device(self.key_code, key, what="KIVI dequantization")
             self._restore("uc_kivi_restore", device, key, value, 0, self.quantized_tokens, 0,
                           dense[0].data_ptr(), dense[1].data_ptr(), self.residual_tokens)

@@ -326,6 +326,33 @@ def test_finer_splits_hand_over_fp32_partials(device, bits, group, hq, lq, lengt
     assert torch.equal(out, one.outputs[0]) and torch.equal(lse, one.lses[0])
 
 
+def test_finer_splits_in_a_graph(device):
+    # a captured run of finer splits, replayed over changing queries with eager
+    # work in between, gives what the eager run gives
+    from unicache_amd.storage.decode import KiviDecodeBatch
+
+    caches = [_pair(t, 220 + i, 2, 32, 128, device)[0] for i, t in enumerate((2500, 700))]
+    qs = [queries(1, seed=230 + i).to(device) for i in range(2)]
+    batch = KiviDecodeBatch(caches, qs)
+    batch.run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        batch.run()
+    for step in range(4):
+        for i, q in enumerate(qs):
+            q.copy_(queries(1, seed=240 + 2 * step + i))
+        batch.run()
+        want = [x.clone() for x in batch.outputs + batch.lses]
+        for x in batch.outputs + batch.lses:
+            x.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, exp in zip(batch.outputs + batch.lses, want):
+            assert torch.equal(x, exp), f"replay {step}"
+
+
 def test_decode_combine_of_many_splits(device):
     # one packed segment and 7 dense ones of up to 13 splits at 4 query rows per
     # KV head: 112 splits, the 16 parts a combine block takes at most
